@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 
 import g3d_amd
+import refpy
 
 pytestmark = pytest.mark.gpu
 LAMBDA_TEST = 10e-6          # the reference tests' unit system (Config::base_units(10e-6))
@@ -321,6 +322,7 @@ def ionization_run(el, Z0, Zmax, mobile, a0):
     return frac, n
 
 
+@pytest.mark.skipif(not refpy.available(), reason="oracle/_ref not built")
 def test_field_ionization_rate_equations():
     """Monte Carlo ADK ionization against the rate equations (tests/test_ionization.cpp:83-90): hydrogen, fixed
     atoms, a0 = 0.01; N5+ -> N6+ -> N7+, mobile ions, a0 = 2"""

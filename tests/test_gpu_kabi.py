@@ -13,7 +13,7 @@ import g3d_amd
 import refpy
 from decks import bunch_deck, particle_parity, plasma_deck
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not refpy.available(), reason="oracle/_ref not built")]
 D = g3d_amd.DevArray
 
 
