@@ -1028,41 +1028,63 @@ void Sim::load_plasma(double s0, double s1) {
     parts_copy(strmA.view(), strmB.view(&strmA), nstrm);
 }
 
-// The common case on the device: Fourier y, tiled, electrons only and every lattice point loaded (the density is
-// positive on the whole box: no radial cut inside it, no negative channel, a positive longitudinal factor).  The
-// list is then the host loader's, regrouped by tile, with the same values and ids.
+// The common case on the device: a tiled list with every lattice point loaded (the density is positive on the whole
+// box: no radial cut inside it, no negative channel, a positive longitudinal factor), electrons and ion species on
+// either y grid.  The list is then the host loader's, regrouped by tile, with the same values and ids (512 x 386 free-hand
+// cells with hydrogen and nitrogen, 1.2 million entries: the host loader and its copy took about 0.2 s of a step).
 bool Sim::load_plasma_device(double s0, double s1) {
     const char* e = getenv("G3D_HOST_LATTICE");                 // 1: always the host loader (for comparisons)
-    if ((e && atoi(e) > 0) || !yf || tiles.ntile <= 0 || !cfg.free_electrons || !cfg.plasma_on || cfg.n0 <= 0) return false;
-    for (const auto& is : cfg.ions) if (cfg.loaded(is)) return false;
+    if ((e && atoi(e) > 0) || tiles.ntile <= 0 || !cfg.plasma_on || cfg.n0 <= 0) return false;
     const double zmid = 0.5 * (s0 + s1);
     const double f = cfg.plasma_zfactor(zmid);
     if (!(f > 0) || (cfg.parabolic && !(cfg.channel_depth >= 0))) return false;
-    const double xm = std::max(std::fabs(X0), std::fabs(X0 + cfg.Lx)), ym = std::max(std::fabs(Y0), std::fabs(Y0 + cfg.Ly));
-    if (!(xm * xm + ym * ym < 0.99 * cfg.r_max * cfg.r_max)) return false;      // no point beyond the radial cut
     const int nx = cfg.nx, ny = cfg.ny, px = cfg.ppc_x, py = cfg.ppc_y;
     if (px < 1 || py < 1) return false;
-    LatticeArgs L;
-    L.nx = nx; L.ny = ny; L.px = px; L.py = py; L.TX = tiles.TX; L.TY = tiles.TY; L.ntx = tiles.ntx;
+    const double ya = yf ? Y0 : cfg.ynode[0] + Y0, yb = yf ? Y0 + cfg.Ly : cfg.ynode[ny] + Y0;
+    const double xm = std::max(std::fabs(X0), std::fabs(X0 + cfg.Lx)), ym = std::max(std::fabs(ya), std::fabs(yb));
+    if (!(xm * xm + ym * ym < 0.99 * cfg.r_max * cfg.r_max)) return false;      // no point beyond the radial cut
+    LatticeArgs L{};
+    L.nsp = 0;
+    long levels = 0;                   // electrons that the ions of a lattice point can free
+    if (cfg.free_electrons) L.sp[L.nsp++] = LatticeSpecies{-1, -1, 1.0, SP_PLASMA};
+    for (size_t k = 0; k < cfg.ions.size(); ++k) {
+        const g3d_ion& is = cfg.ions[k];
+        if (!cfg.loaded(is)) continue;
+        if (L.nsp >= kLatticeSpecies) return false;
+        L.sp[L.nsp++] = LatticeSpecies{double(is.Z0), is.Z0 / is.mass, is.atoms, SP_ION + int(k)};
+        if (is.ionization) levels += is.Zmax - is.Z0;
+    }
+    if (!L.nsp) return false;
+    L.nx = nx; L.px = px; L.py = py; L.TX = tiles.TX; L.TY = tiles.TY; L.ntx = tiles.ntx;
     L.parabolic = cfg.parabolic;
-    L.per_tile = long(tiles.TX) * tiles.TY * px * py;
+    L.j0 = yf ? 0 : 1; L.j1 = yf ? ny : ny - 1;                 // no plasma in the cells at the walls
+    L.yn = yf ? nullptr : yn.data();
     L.dx = dx; L.dy = dy; L.X0 = X0; L.Y0 = Y0; L.zf = cfg.zeta[N - 1]; L.s0 = s0; L.Delta = s1 - s0;
     L.n0 = cfg.n0; L.f = f; L.channel_depth = cfg.channel_depth; L.r_channel = cfg.r_channel;
     const unsigned long long id0 = (unsigned long long)(istep + 1) << 32;
     id0_ = id0;
     L.id0 = id0;
-    const long fresh = L.per_tile * tiles.ntile;
+    std::vector<long> off(tiles.ntile + 1, 0);
+    for (long t = 0; t < tiles.ntile; ++t) {
+        const int jt = int(t / tiles.ntx) * tiles.TY;
+        const int rows = std::min(jt + tiles.TY, L.j1) - std::max(jt, L.j0);
+        off[t + 1] = off[t] + long(std::max(rows, 0)) * tiles.TX * px * py * L.nsp;
+    }
+    const long fresh = off[tiles.ntile];
     const long total = fresh + long(joining_.size());
     fresh_last = fresh;
-    std::vector<long> off(tiles.ntile + 1);
-    for (long t = 0; t <= tiles.ntile; ++t) off[t] = t * L.per_tile;
     tile_off.from_host(off.data(), 0, off.size());
+    L.off = tile_off.data();
     n_tiled = fresh;
     tiles.n_tiled = n_tiled;
     nstrm = total;
-    born_cap = 0;
-    ensure_strm(size_t(total));
-    plasma_lattice(L, strmA.view(), strmB.view(&strmA), fresh);
+    born_cap = fresh / L.nsp * levels;
+    for (const auto& p : joining_)
+        if (is_ion(p.sp) && cfg.ions[p.sp - SP_ION].ionization)
+            born_cap += cfg.ions[p.sp - SP_ION].Zmax - std::lround(p.q);
+    if (born_cap > 0 && born.cap < size_t(born_cap)) born.resize(size_t(born_cap));
+    ensure_strm(size_t(total) + size_t(born_cap));
+    plasma_lattice(L, strmA.view(), strmB.view(&strmA), tiles.ntile);
     if (!joining_.empty()) {      // trapped particles too slow to join the beam stream again, waiting (alive 6)
         std::vector<g3d_particle> v(joining_);
         for (auto& p : v) p.alive = 6;
@@ -1414,12 +1436,9 @@ void Sim::march_plasma(double s0, double s1) {
     }
     // trapped particles (alive 5): fast ones join the beam list, slow ones stream again in the next step
     std::vector<g3d_particle> sv;
-    bool need_all = false;
-    for (const auto& is : cfg.ions) need_all = need_all || is.ionization;
-    if (need_all) sv = host_strm();
-    else {
+    {
         counters.zero();
-        if (aos.size() < size_t(std::max<long>(nstrm, 1))) aos.resize(size_t(std::max<long>(nstrm, 1)));
+        if (aos.size() < std::max<size_t>(strmA.cap, 1)) aos.resize(std::max<size_t>(strmA.cap, 1));
         if (aos_idx.size() < aos.size()) aos_idx.resize(aos.size());
         collect_alive(strmA.view(), nstrm, 5, aos.data(), aos_idx.data(), counters.data() + 1, long(aos.size()));
         int cnt = 0;
@@ -1438,18 +1457,26 @@ void Sim::march_plasma(double s0, double s1) {
             for (int k : ord) sv.push_back(t[k]);
         }
     }
-    std::vector<g3d_particle> add;
     for (auto& h : ion_stats) h.clear();
-    for (auto& p : sv) {
-        if (is_ion(p.sp) && cfg.ions[p.sp - SP_ION].ionization) {
-            const auto& is = cfg.ions[p.sp - SP_ION];
-            std::vector<double>& h = ion_stats[p.sp - SP_ION];
-            if (h.empty()) h.assign(is.Zmax + 2, 0.0);
-            const int Z = int(std::lround(p.q));
-            if (p.alive == 1) h[Z] += p.w;
-            h[is.Zmax + 1] += (Z - is.Z0) * p.w;
+    {   // the charge states of the ionizing species
+        IonStatArgs ia{};
+        for (int k = 0; k < 4; ++k) {
+            const bool on = k < int(cfg.ions.size()) && cfg.ions[k].ionization && nstrm > 0;
+            ia.s[k] = IonStatSpecies{on ? ia.nslot : -1, on ? cfg.ions[k].Z0 : 0, on ? cfg.ions[k].Zmax : 0};
+            if (on) ia.nslot += cfg.ions[k].Zmax + 2;
         }
-        if (p.alive != 5) continue;
+        if (ia.nslot > 0) {
+            if (ion_part.size() < size_t(kIonStatBlocks + 1) * ia.nslot) ion_part.resize(size_t(kIonStatBlocks + 1) * ia.nslot);
+            double* out = ion_part.data() + size_t(kIonStatBlocks) * ia.nslot;
+            ion_statistics(ia, strmA.view(), nstrm, ion_part.data(), out);
+            std::vector<double> v(static_cast<size_t>(ia.nslot));
+            ion_part.to_host(v.data(), size_t(kIonStatBlocks) * ia.nslot, v.size());
+            for (size_t k = 0; k < ion_stats.size() && k < 4; ++k)
+                if (ia.s[k].slot >= 0) ion_stats[k].assign(v.begin() + ia.s[k].slot, v.begin() + ia.s[k].slot + ia.s[k].Zmax + 2);
+        }
+    }
+    std::vector<g3d_particle> add;
+    for (auto& p : sv) {
         const double gg = std::sqrt(1 + p.px * p.px + p.py * p.py + p.pz * p.pz);
         p.z = s1;
         if (p.pz / gg >= cfg.vz_beam) {

@@ -206,6 +206,7 @@ public:
     DevBuf<long> tile_off;
     DevBuf<int> bin_idx, bin_cnt, bin_cur;   // binning of the live list by current tile
     DevBuf<double> slab;
+    DevBuf<double> ion_part;          // partial sums of the ion statistics
     long n_tiled = 0;
     unsigned long long id0_ = 0;
 

@@ -160,20 +160,33 @@ void count_alive(Parts p, long n, int code, int* count);
 void parts_from_aos(const g3d_particle* in, Parts p, long n);
 void parts_to_aos(Parts p, g3d_particle* out, long n);
 void parts_copy(Parts src, Parts dst, long n);
-// The fresh plasma of a step on the device (src/sim_plasma.cpp:43-90 for electrons only, Fourier y, every lattice
-// point loaded): lattice points in tile order (tiles of TX x TY cells, per_tile = TX TY px py points each; inside a
-// tile the sub-position (b2, a2) outermost, then the cells j-major, so that the 64 lanes of a wave push electrons
-// of 64 different cells and their deposits into the tile's LDS window meet no same-address atomics: the stream
-// kernel runs 8 % faster than with the points of a cell adjacent), each with the host loader's values and its id in
-// the reference's order, id0 + ((j nx + i) py + b2) px + a2.  The density is n0 f g with the longitudinal factor f of the step and the
-// channel factor g.
+// The fresh plasma of a step on the device (src/sim_plasma.cpp:43-90, every lattice point loaded): electrons and
+// ion species, either y grid, in tile order (tiles of TX x TY cells; off[t]: the first entry of tile t).  Inside a
+// tile the species is outermost, then the sub-position (b2, a2), then the cells j-major: the 64 lanes of a wave push
+// particles of one species in 64 different cells, so they take one branch and their deposits into the tile's LDS
+// window meet no same-address atomics (electrons only: the stream kernel 8 % faster than with the points of a cell
+// adjacent; with hydrogen and nitrogen on the free-hand grid see k_stream_halfcell).  Every entry has the host
+// loader's values and its id in the reference's order, id0 + (((j - j0) nx + i) py + b2) px + a2) nsp + k.  The
+// density is n0 f g with the longitudinal factor f of the step and the channel factor g.
+struct LatticeSpecies { double q, qm, atoms; int sp; };    // weight: atoms times the electron's (electrons: 1)
+constexpr int kLatticeSpecies = 5;
 struct LatticeArgs {
-    int nx, ny, px, py, TX, TY, ntx, parabolic;
-    long per_tile;
+    int nx, px, py, TX, TY, ntx, parabolic, nsp;
+    int j0, j1;                       // the loaded rows of cells (free-hand y: without those at the walls)
+    const double* yn;                 // free-hand y: the node table; null: rows of dy
+    const long* off;
     double dx, dy, X0, Y0, zf, s0, Delta, n0, f, channel_depth, r_channel;
     unsigned long long id0;
+    LatticeSpecies sp[kLatticeSpecies];
 };
-void plasma_lattice(const LatticeArgs& L, Parts A, Parts B, long n);
+void plasma_lattice(const LatticeArgs& L, Parts A, Parts B, long ntile);
+// The ion statistics of a step (src/sim_plasma.cpp:438-446) summed on the device in a fixed tree order: for the
+// species of spec[0 .. nspec) (code SP_ION + k at slot[k] of out; slot -1: none) the weight of each charge state of
+// the ions still streaming, then the freed charge.  part: kIonStatBlocks nslot doubles of scratch
+constexpr int kIonStatBlocks = 1024;
+struct IonStatSpecies { int slot, Z0, Zmax; };
+struct IonStatArgs { IonStatSpecies s[4]; int nslot; };
+void ion_statistics(const IonStatArgs& a, Parts p, long n, double* part, double* out);
 void parts_shift(Parts p, long n, double sx, double sy);
 
 // ---------------------------------------------------------------- spectra and fields (Fourier y)

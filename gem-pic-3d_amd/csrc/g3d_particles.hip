@@ -689,15 +689,17 @@ __global__ void __launch_bounds__(kT) k_bin_scatter(Parts S, long n, TileGeom tg
     if (t >= 0) idx[lbase[t] + r] = int(i);
 }
 __global__ void k_append_born(Parts b, const int* bcnt, Parts p0, Parts p1, long base, long cap) {
-    const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
     const long cnt = *bcnt;
-    if (i >= cnt || base + i >= cap) return;
-    const long d = base + i;
-    for (Parts* t : {&p0, &p1}) {
-        t->x[d] = b.x[i]; t->y[d] = b.y[i]; t->zeta[d] = b.zeta[i]; t->px[d] = b.px[i]; t->py[d] = b.py[i];
-        t->pz[d] = b.pz[i]; t->z[d] = b.z[i]; t->q[d] = b.q[i]; t->qm[d] = b.qm[i]; t->alive[d] = b.alive[i];
+    // a few workgroups stride over the count (a grid for the whole capacity, up to Zmax times the ions, only exits)
+    for (long i = long(blockIdx.x) * blockDim.x + threadIdx.x; i < cnt && base + i < cap;
+         i += long(gridDim.x) * blockDim.x) {
+        const long d = base + i;
+        for (Parts* t : {&p0, &p1}) {
+            t->x[d] = b.x[i]; t->y[d] = b.y[i]; t->zeta[d] = b.zeta[i]; t->px[d] = b.px[i]; t->py[d] = b.py[i];
+            t->pz[d] = b.pz[i]; t->z[d] = b.z[i]; t->q[d] = b.q[i]; t->qm[d] = b.qm[i]; t->alive[d] = b.alive[i];
+        }
+        p0.w[d] = b.w[i]; p0.sp[d] = b.sp[i]; p0.id[d] = b.id[i]; p0.rem[d] = 0;
     }
-    p0.w[d] = b.w[i]; p0.sp[d] = b.sp[i]; p0.id[d] = b.id[i]; p0.rem[d] = 0;
 }
 
 // ---------------------------------------------------------------- list tools
@@ -869,8 +871,8 @@ void bin_tiles(Parts S, Parts D, long n, const TileGeom& tg, double dx, double d
 }
 void append_born(Parts born, const int* bcnt, Parts p0, Parts p1, long base, long cap) {
     if (cap <= base) return;
-    hipLaunchKernelGGL(k_append_born, dim3(blocks_for(cap - base, kT)), dim3(kT), 0, stream(), born, bcnt, p0, p1, base,
-                       cap);
+    const unsigned nb = std::min(blocks_for(cap - base, kT), 128u);
+    hipLaunchKernelGGL(k_append_born, dim3(nb), dim3(kT), 0, stream(), born, bcnt, p0, p1, base, cap);
     launch_check("append born");
 }
 void bunch_centroid(Parts p, long np, double X0, double Y0, double* out3) {
@@ -901,37 +903,83 @@ void parts_to_aos(Parts p, g3d_particle* out, long n) {
     hipLaunchKernelGGL(k_to_aos, dim3(blocks_for(n, kT)), dim3(kT), 0, stream(), p, out, n);
     launch_check("particles to AoS");
 }
-// the fresh plasma lattice of a step, generated in tile order (see LatticeArgs); both list buffers
-__global__ void k_lattice(LatticeArgs L, Parts A, Parts B, long n) {
-    const long g = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (g >= n) return;
-    const int pp = L.px * L.py;
-    const long t = g / L.per_tile, r = g - t * L.per_tile;
-    const long cpt = L.per_tile / pp;                // cells of a tile: the sub-position outermost
-    const int sub = int(r / cpt);
-    const long c = r - sub * cpt;
-    const int jl = int(c / L.TX), il = int(c - long(jl) * L.TX);
-    const int b2 = sub / L.px, a2 = sub - b2 * L.px;
+// the fresh plasma lattice of a step, generated in tile order (see LatticeArgs), one workgroup per tile; both list
+// buffers
+__global__ void __launch_bounds__(kT) k_lattice(LatticeArgs L, Parts A, Parts B) {
+    const long t = blockIdx.x;
     const int tx = int(t % L.ntx), ty = int(t / L.ntx);
-    const int j = ty * L.TY + jl, i = tx * L.TX + il;
-    // the host loader's formulas and operation order (src/sim_plasma.cpp:62-64)
-    const double y0 = j * L.dy, hy = L.dy;
-    const double x = (i + (a2 + 0.5) / L.px) * L.dx;
-    const double y = y0 + (b2 + 0.5) / L.py * hy;
-    const double X = x + L.X0, Y = y + L.Y0, r2 = X * X + Y * Y;
-    const double gch = L.parabolic ? 1 + L.channel_depth * r2 / (L.r_channel * L.r_channel) : 1.0;
-    const double dens = L.f * gch > 0 ? L.n0 * L.f * gch : 0.0;
-    const double w = dens * L.dx * hy * L.Delta / (L.px * L.py);
-    A.x[g] = x; A.y[g] = y; A.zeta[g] = L.zf; A.px[g] = 0; A.py[g] = 0; A.pz[g] = 0; A.w[g] = w; A.rem[g] = 0;
-    A.z[g] = L.s0; A.q[g] = -1; A.qm[g] = -1; A.alive[g] = 1; A.sp[g] = SP_PLASMA;
-    A.id[g] = L.id0 + (((unsigned long long)j * L.nx + i) * L.py + b2) * L.px + a2;
-    B.x[g] = x; B.y[g] = y; B.zeta[g] = L.zf; B.px[g] = 0; B.py[g] = 0; B.pz[g] = 0; B.z[g] = L.s0; B.q[g] = -1;
-    B.qm[g] = -1; B.alive[g] = 1;
+    const int jt = ty * L.TY, ja = jt < L.j0 ? L.j0 : jt;      // the tile's first loaded row
+    const long lo = L.off[t], n = L.off[t + 1] - lo;
+    const int pp = L.px * L.py;
+    const int per = int(n / (L.nsp * pp));                     // cells of the tile
+    for (int r = threadIdx.x; r < n; r += blockDim.x) {
+        const int k = r / (pp * per), rk = r - k * pp * per;
+        const int sub = rk / per, c = rk - sub * per;
+        const int jl = c / L.TX, il = c - jl * L.TX;
+        const int b2 = sub / L.px, a2 = sub - b2 * L.px;
+        const int j = ja + jl, i = tx * L.TX + il;
+        // the host loader's formulas and operation order (src/sim_plasma.cpp:62-64)
+        const double y0 = L.yn ? L.yn[j] : j * L.dy, hy = L.yn ? L.yn[j + 1] - L.yn[j] : L.dy;
+        const double x = (i + (a2 + 0.5) / L.px) * L.dx;
+        const double y = y0 + (b2 + 0.5) / L.py * hy;
+        const double X = x + L.X0, Y = y + L.Y0, r2 = X * X + Y * Y;
+        const double gch = L.parabolic ? 1 + L.channel_depth * r2 / (L.r_channel * L.r_channel) : 1.0;
+        const double dens = L.f * gch > 0 ? L.n0 * L.f * gch : 0.0;
+        const LatticeSpecies S = L.sp[k];
+        const double w = S.atoms * (dens * L.dx * hy * L.Delta / (L.px * L.py));
+        const long g = lo + r;
+        A.x[g] = x; A.y[g] = y; A.zeta[g] = L.zf; A.px[g] = 0; A.py[g] = 0; A.pz[g] = 0; A.w[g] = w; A.rem[g] = 0;
+        A.z[g] = L.s0; A.q[g] = S.q; A.qm[g] = S.qm; A.alive[g] = 1; A.sp[g] = S.sp;
+        A.id[g] = L.id0 + ((((unsigned long long)(j - L.j0) * L.nx + i) * L.py + b2) * L.px + a2) * L.nsp + k;
+        B.x[g] = x; B.y[g] = y; B.zeta[g] = L.zf; B.px[g] = 0; B.py[g] = 0; B.pz[g] = 0; B.z[g] = L.s0; B.q[g] = S.q;
+        B.qm[g] = S.qm; B.alive[g] = 1;
+    }
 }
-void plasma_lattice(const LatticeArgs& L, Parts A, Parts B, long n) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_lattice, dim3(blocks_for(n, kT)), dim3(kT), 0, stream(), L, A, B, n);
+void plasma_lattice(const LatticeArgs& L, Parts A, Parts B, long ntile) {
+    if (ntile <= 0) return;
+    hipLaunchKernelGGL(k_lattice, dim3(unsigned(ntile)), dim3(kT), 0, stream(), L, A, B);
     launch_check("plasma lattice");
+}
+
+// ion statistics: every lane its own sums in LDS ([slot][lane]), then a tree over the lanes of the workgroup, then
+// the workgroups in order
+constexpr int kIonStatLanes = 64;
+__global__ void __launch_bounds__(kIonStatLanes) k_ion_stats(IonStatArgs a, Parts p, long n, double* part) {
+    extern __shared__ double ist[];
+    const int t = threadIdx.x;
+    for (int s = 0; s < a.nslot; ++s) ist[s * kIonStatLanes + t] = 0;
+    for (long i = long(blockIdx.x) * kIonStatLanes + t; i < n; i += long(gridDim.x) * kIonStatLanes) {
+        const int sp = p.sp[i];
+        if (sp < SP_ION || sp >= SP_ION + 4) continue;
+        const IonStatSpecies S = a.s[sp - SP_ION];
+        if (S.slot < 0) continue;
+        const int Z = int(floor(p.q[i] + 0.5));
+        const double w = p.w[i];
+        if (p.alive[i] == 1 && Z >= 0 && Z <= S.Zmax) ist[(S.slot + Z) * kIonStatLanes + t] += w;
+        ist[(S.slot + S.Zmax + 1) * kIonStatLanes + t] += (Z - S.Z0) * w;
+    }
+    __syncthreads();
+    for (int o = kIonStatLanes / 2; o > 0; o >>= 1) {
+        if (t < o)
+            for (int s = 0; s < a.nslot; ++s) ist[s * kIonStatLanes + t] += ist[s * kIonStatLanes + t + o];
+        __syncthreads();
+    }
+    for (int s = t; s < a.nslot; s += kIonStatLanes) part[long(blockIdx.x) * a.nslot + s] = ist[s * kIonStatLanes];
+}
+__global__ void k_ion_stats_final(const double* part, int nslot, int nb, double* out) {
+    const int s = threadIdx.x;
+    if (s >= nslot) return;
+    double v = 0;
+    for (int b = 0; b < nb; ++b) v += part[long(b) * nslot + s];
+    out[s] = v;
+}
+void ion_statistics(const IonStatArgs& a, Parts p, long n, double* part, double* out) {
+    if (a.nslot <= 0) return;
+    if (a.nslot > 128) throw std::runtime_error("ion statistics: too many charge states");
+    const size_t lds = size_t(a.nslot) * kIonStatLanes * sizeof(double);
+    hipLaunchKernelGGL(k_ion_stats, dim3(kIonStatBlocks), dim3(kIonStatLanes), lds, stream(), a, p, n, part);
+    hipLaunchKernelGGL(k_ion_stats_final, dim3(1), dim3(128), 0, stream(), part, a.nslot, kIonStatBlocks, out);
+    launch_check("ion statistics");
 }
 void parts_copy(Parts s, Parts d, long n) {
     if (n <= 0) return;
