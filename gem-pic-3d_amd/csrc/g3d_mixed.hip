@@ -94,12 +94,12 @@ __device__ __forceinline__ void boris_d(double& ux, double& uy, double& uz, cons
 constexpr int kFwNode = 12, kDepNode = 5;
 struct WinD {
     double* lds;              // kDepNode doubles per node
-    const float4* fld;        // 3 float4 per node, or null
+    const float4* fld;        // 3 float4 per node
     int x0, y0, WX, WY, fl;
 };
 
 // E, B at a point: the tile's field window when the stencil and the slice pair are in it, else F
-__device__ __forceinline__ void gather_d(const FieldView& c, const InvD& iv, const WinD* w, double x, double y,
+__device__ __forceinline__ void gather_d(const FieldView& c, const InvD& iv, const WinD& w, double x, double y,
                                          double zeta, double E[3], double B[3]) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) { E[k] = 0; B[k] = 0; }
@@ -117,15 +117,15 @@ __device__ __forceinline__ void gather_d(const FieldView& c, const InvD& iv, con
     for (int j = 0; j < 3; ++j)
 #pragma unroll
         for (int i = 0; i < 3; ++i) wt[3 * j + i] = wx[i] * wn[j];
-    if (w && w->fld && fl == w->fl) {
-        const int u0 = wrap_index(i0 - 1 - w->x0, c.nx), v0 = wrap_index(j0 - 1 - w->y0, c.ny);
-        if (u0 + 2 < w->WX && v0 + 2 < w->WY) {
+    if (w.WX && fl == w.fl) {
+        const int u0 = wrap_index(i0 - 1 - w.x0, c.nx), v0 = wrap_index(j0 - 1 - w.y0, c.ny);
+        if (u0 + 2 < w.WX && v0 + 2 < w.WY) {
             double s0[6] = {0, 0, 0, 0, 0, 0}, s1[6] = {0, 0, 0, 0, 0, 0};
 #pragma unroll
             for (int j = 0; j < 3; ++j)
 #pragma unroll
                 for (int i = 0; i < 3; ++i) {
-                    const float4* q = w->fld + 3 * ((v0 + j) * w->WX + u0 + i);
+                    const float4* q = w.fld + 3 * ((v0 + j) * w.WX + u0 + i);
                     const float4 a = q[0], b = q[1], d = q[2];
                     const double t = wt[3 * j + i];
                     s0[0] += t * double(a.x); s0[1] += t * double(a.y); s0[2] += t * double(a.z);
@@ -164,7 +164,7 @@ __device__ __forceinline__ void gather_d(const FieldView& c, const InvD& iv, con
 // TSC deposit of f v into the current window (FP64 sums) or, outside it, into the FP32 current planes with float
 // atomics (src/sim_stream.hpp:33-48); f includes the inverse area factor.  The charge density planes (rho-, rho+)
 // only when rho (their one reader, the density lines, takes the last pass's)
-__device__ __forceinline__ void sdeposit_d(const StreamArgs& c, const InvD& iv, float* J, const WinD* win, double x,
+__device__ __forceinline__ void sdeposit_d(const StreamArgs& c, const InvD& iv, float* J, const WinD& win, double x,
                                            double y, double f, double vx, double vy, double vz, bool rho) {
     const FieldView& P = c.fv;
     double wx[3], wn[3];
@@ -174,14 +174,14 @@ __device__ __forceinline__ void sdeposit_d(const StreamArgs& c, const InvD& iv, 
     const bool mv = vx != 0 || vy != 0 || vz != 0;
 #pragma unroll
     for (int k = 0; k < 3; ++k) wx[k] *= f;
-    if (win) {
-        const int u0 = wrap_index(i0 - 1 - win->x0, P.nx), v0 = wrap_index(j0 - 1 - win->y0, P.ny);
-        if (u0 + 2 < win->WX && v0 + 2 < win->WY) {
+    if (win.WX) {
+        const int u0 = wrap_index(i0 - 1 - win.x0, P.nx), v0 = wrap_index(j0 - 1 - win.y0, P.ny);
+        if (u0 + 2 < win.WX && v0 + 2 < win.WY) {
 #pragma unroll
             for (int v = 0; v < 3; ++v)
 #pragma unroll
                 for (int u = 0; u < 3; ++u) {
-                    double* L = win->lds + kDepNode * ((v0 + v) * win->WX + (u0 + u));
+                    double* L = win.lds + kDepNode * ((v0 + v) * win.WX + (u0 + u));
                     const double ww = wx[u] * wn[v];
                     if (mv) {
                         atomicAdd(L, ww * vx);
@@ -237,7 +237,7 @@ __device__ __forceinline__ HalfCellD half_cell(const StreamArgs& c, int rho) {
 // LASER: the deck has the analytic laser (its evaluation would otherwise set the register budget of every launch)
 template <bool LASER>
 __device__ __forceinline__ void stream_one_mixed(const StreamArgs& c, const HalfCellD& hc, const InvD& iv, float* J,
-                                                 const WinD* win, const MState& s, Parts D, long i) {
+                                                 const WinD& win, const MState& s, Parts D, long i) {
     const double zn = hc.zn, zn1 = hc.zn1, h = hc.h;
     double x = s.x, y = s.y, zeta = s.zeta, z = s.z;
     const double px = s.px, py = s.py, pz = s.pz;
@@ -297,14 +297,18 @@ __device__ __forceinline__ void stream_one_mixed(const StreamArgs& c, const Half
     zeta = zeta_end;
     // the streaming current q w dt / (Delta h dx) of the half-cell
     const double qw = q * w;
-    const double f = qw * hc.iq * dt;
-    if (f != 0) sdeposit_d(c, iv, J, win, 0.5 * (xo + x), 0.5 * (yo + y), f, vx, vy, vz, hc.rho);
-    if (trapped) {
-        alive = 5;
-        const double vze = uz * ig1;
-        // joins the beam list: its beam current q w / (h dx v_z) of level s1 from now on
-        if (vze >= c.vz_beam) sdeposit_d(c, iv, J, win, x, y, qw * hc.iqb * rcp_d(vze), ux * ig1, uy * ig1, vze, hc.rho);
+    double f = qw * hc.iq * dt, xd = 0.5 * (xo + x), yd = 0.5 * (yo + y);
+    const double vze = uz * ig1;
+    // a trapped electron that joins the beam list: its beam current q w / (h dx v_z) of level s1 from now on, after
+    // the streaming current (one copy of the deposit in the code)
+    const bool join = trapped && vze >= c.vz_beam;
+#pragma unroll 1
+    for (int d = 0;; ++d) {
+        if (f != 0 || d) sdeposit_d(c, iv, J, win, xd, yd, f, vx, vy, vz, hc.rho);
+        if (d || !join) break;
+        xd = x; yd = y; f = qw * hc.iqb * rcp_d(vze); vx = ux * ig1; vy = uy * ig1; vz = vze;
     }
+    if (trapped) alive = 5;
     store(ux, uy, uz);
 }
 
@@ -315,35 +319,42 @@ k_stream_mixed(StreamArgs c, float* J, float* slab, Parts S, Parts D, long n, Ti
     extern __shared__ double2 wind2[];
     const long b = blockIdx.x;
     const long nt = tg.ntile + tg.max_extra;
-    if (b < nt) {
-        // workgroups b < max_extra: the further chunks of dense tiles (first, so that they run beside the first
-        // chunks), added to J with atomics; then tile b - max_extra's first chunk, written to its slab
-        long t, lo, hi;
-        const bool extra = b < tg.max_extra;
+    // workgroups b < max_extra: the further chunks of dense tiles (first, so that they run beside the first
+    // chunks), added to J with atomics; then tile b - max_extra's first chunk, written to its slab; then the untiled
+    // rest, one electron per lane
+    const bool tiled = b < nt, extra = b < tg.max_extra;
+    long t = 0, lo, hi;
+    if (!tiled) {
+        lo = tg.n_tiled + (b - nt) * blockDim.x;
+        hi = lo + blockDim.x < n ? lo + blockDim.x : n;
+    } else {
         if (!extra) {
             t = b - tg.max_extra;
             if (tg.xcd) t = row_block(int(t), int(tg.ntile), 1);
-            lo = tg.off[t]; hi = tg.off[t + 1];
-        }
-        else {
+            lo = tg.off[t];
+        } else {
             if (b >= tg.xcount[0]) return;
-            t = tg.xtile[b]; lo = tg.xstart[b]; hi = tg.off[t + 1];
+            t = tg.xtile[b]; lo = tg.xstart[b];
         }
+        hi = tg.off[t + 1];
         if (tg.chunk > 0 && hi - lo > tg.chunk) hi = lo + tg.chunk;
-        // the range, this lane's first particle and its state first: their dependent loads overlap the loads of
-        // the field window
-        long k = lo + threadIdx.x;
-        long i = k < hi ? (tg.idx ? long(tg.idx[k]) : k) : 0;
-        MState st{};
-        if (k < hi) st = load_mstate(S, i);
-        const int pl = tg.WX * tg.WY;
-        const int wn = kDepNode * pl;
-        const int tx = int(t % tg.ntx), ty = int(t / tg.ntx);
-        const int x0 = tx * tg.TX - 1 - tg.M, y0 = ty * tg.TY - 1 - tg.M;
-        const FieldView& F = c.fv;
-        const int fl = c.n - F.a;
-        float4* fw = reinterpret_cast<float4*>(wind2);
-        double* dep = reinterpret_cast<double*>(fw + 3 * pl);
+    }
+    // the range, this lane's first particle and its state first: their dependent loads overlap the loads of
+    // the field window
+    const int* idx = tiled ? tg.idx : nullptr;
+    long k = lo + threadIdx.x;
+    long i = k < hi ? (idx ? long(idx[k]) : k) : 0;
+    MState st{};
+    if (k < hi) st = load_mstate(S, i);
+    const int pl = tg.WX * tg.WY;
+    const int wn = kDepNode * pl;
+    const int tx = tiled ? int(t % tg.ntx) : 0, ty = tiled ? int(t / tg.ntx) : 0;
+    const int x0 = tx * tg.TX - 1 - tg.M, y0 = ty * tg.TY - 1 - tg.M;
+    const FieldView& F = c.fv;
+    const int fl = c.n - F.a;
+    float4* fw = reinterpret_cast<float4*>(wind2);
+    double* dep = reinterpret_cast<double*>(fw + 3 * pl);
+    if (tiled) {
         for (int r = threadIdx.x; r < wn; r += blockDim.x) dep[r] = 0;
         if (F.self)      // one node per lane: its 12 values from the 6 component planes of slices fl, fl + 1
             for (int r = threadIdx.x; r < pl; r += blockDim.x) {
@@ -362,19 +373,21 @@ k_stream_mixed(StreamArgs c, float* J, float* slab, Parts S, Parts D, long n, Ti
                     fw[3 * r + k] = make_float4(q[4 * k], q[4 * k + 1], q[4 * k + 2], q[4 * k + 3]);
             }
         __syncthreads();
-        WinD w{dep, F.self ? fw : nullptr, x0, y0, tg.WX, tg.WY, fl};
-        const InvD iv{1.0 / F.dx, 1.0 / F.dy};
-        const HalfCellD hc = half_cell(c, rho);
-        unsigned cnt = 0;
-        while (k < hi) {
-            cnt += pushed_through(st.alive, st.zeta, hc.zn);
-            stream_one_mixed<LASER>(c, hc, iv, J, &w, st, D, i);
-            k += blockDim.x;
-            if (k < hi) {
-                i = tg.idx ? long(tg.idx[k]) : k;
-                st = load_mstate(S, i);
-            }
+    }
+    const WinD w{dep, fw, x0, y0, tiled ? tg.WX : 0, tg.WY, fl};
+    const InvD iv{1.0 / F.dx, 1.0 / F.dy};
+    const HalfCellD hc = half_cell(c, rho);
+    unsigned cnt = 0;
+    while (k < hi) {
+        cnt += pushed_through(st.alive, st.zeta, hc.zn);
+        stream_one_mixed<LASER>(c, hc, iv, J, w, st, D, i);
+        k += blockDim.x;
+        if (k < hi) {
+            i = idx ? long(idx[k]) : k;
+            st = load_mstate(S, i);
         }
+    }
+    if (tiled) {
         __syncthreads();
         if (!extra && !tg.aflush) {
             float* sl = slab + t * long(wn);
@@ -387,16 +400,6 @@ k_stream_mixed(StreamArgs c, float* J, float* slab, Parts S, Parts D, long n, Ti
                 const long g = long(wrap_index(y0 + vv, F.ny)) * F.nx + wrap_index(x0 + u, F.nx);
                 atomicAdd(&J[cc * F.nk + g], float(v));
             }
-        if (c.npush) add_pushes(c.npush, cnt);
-        return;
-    }
-    const long i = tg.n_tiled + (b - nt) * blockDim.x + threadIdx.x;
-    unsigned cnt = 0;
-    if (i < n) {
-        const HalfCellD hc = half_cell(c, rho);
-        const MState st = load_mstate(S, i);
-        cnt = pushed_through(st.alive, st.zeta, hc.zn);
-        stream_one_mixed<LASER>(c, hc, InvD{1.0 / c.fv.dx, 1.0 / c.fv.dy}, J, nullptr, st, D, i);
     }
     if (c.npush) add_pushes(c.npush, cnt);
 }

@@ -13,92 +13,161 @@ namespace {
 constexpr int kT = 256;
 
 // ---------------------------------------------------------------- streaming particles (src/sim_stream.hpp)
-// LDS windows of a tile, WX x WY nodes from node (x0, y0) (periodic); null for untiled particles:
-//   lds   the 5 current planes of the deposit (double)
-//   fld   the fields of slices fl and fl+1 for the gather (float, [slice][component][WY][WX]), loaded once per
-//         workgroup instead of 108 scattered loads per particle
+// LDS windows of a tile, WX x WY nodes from node (x0, y0) (periodic); WX = 0 for particles without one (one copy of
+// the push in the code for both):
+//   lds   the 5 current planes of the deposit
+//   fld   the fields of slices fl and fl+1 for the gather, node-major (3 float4 per node, win_node),
+//         loaded once per workgroup instead of 108 scattered loads per particle
+//   yn    free-hand y: the nodes y_lo ... y_lo + nyn of the axis, where the locates look first (a bisection of the
+//         table in memory is a chain of dependent loads)
+// The pointers carry the LDS address space: through generic ones the free-hand kernel with ions, which keeps part of
+// its context in memory, read and added by flat instructions (439 us against 350 at 512 x 386 with H and N).
+#define G3D_LDS __attribute__((address_space(3)))
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef G3D_LDS double* ldsd;
 struct Win {
-    double* lds;
-    const float* fld;
-    int x0, y0, WX, WY, fl;
+    ldsd lds;
+    const G3D_LDS f4v* fld;
+    const G3D_LDS double* yn;
+    int x0, y0, WX, WY, fl, y_lo, nyn;
 };
+__device__ __forceinline__ void lds_add(ldsd p, double v) { atomicAdd((double*)p, v); }
+// A node's 12 floats: E_x E_z B_y of slices fl, fl+1 (on the nodes of the free-hand y grid), then E_y B_x B_z of both
+// (on its half-nodes), so that either group is a 16-byte and an 8-byte LDS read
+__device__ __forceinline__ void win_node(G3D_LDS f4v* q, const float* src, long cs, long nk, bool in) {
+    float f[12];
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int comp = g == 0 ? 2 * k : (k == 0 ? 1 : 2 * k + 1);      // 0 2 4, then 1 3 5
+            f[6 * g + k] = in ? src[comp * cs] : 0.0f;
+            f[6 * g + 3 + k] = in ? src[comp * cs + nk] : 0.0f;
+        }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) q[k] = f4v{f[4 * k], f[4 * k + 1], f[4 * k + 2], f[4 * k + 3]};
+}
 
-// E, B from the tile's field window (Fourier y): the same weights and the same order of the sums as gather(), so
-// the values are identical; false when the stencil or the slice pair is not in the window (then the caller
+// tsc_freehand with the cell looked up among the window's nodes first (the cell X[i] <= y < X[i+1] is unique, so the
+// result is the same)
+__device__ __forceinline__ void tsc_freehand_w(const Axis& ax, const Win& w, double y, int jn[3], double wn[3],
+                                               int jh[3], double wh[3]) {
+    int i; double f;
+    if (w.nyn > 0 && w.yn[0] <= y && y < w.yn[w.nyn]) {
+        int lo = 0, hi = w.nyn;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (w.yn[mid] <= y) lo = mid; else hi = mid;
+        }
+        i = w.y_lo + lo; f = (y - w.yn[lo]) / (w.yn[lo + 1] - w.yn[lo]);
+    } else ax.locate(y, i, f);
+    const double xi = i + f;
+    tsc_w(xi, jn, wn);
+    tsc_w(xi - 0.5, jh, wh);
+}
+
+// The TSC stencil of a point in the window: the first node (and half-node) and the weights; false when a row or
+// column that the sums need lies outside it.  Free-hand y: window rows are node indices, rows beyond the walls are
+// skipped (bits of skn, skh)
+struct WinStencil {
+    int kn, kh;
+    unsigned skn, skh;
+    double wx[3], wn[3], wh[3];
+};
+template <int YF>
+__device__ __forceinline__ bool win_stencil(const FieldView& c, const Win& w, double x, double y, WinStencil& s) {
+    int ix[3], jn[3], jh[3];
+    tsc_periodic(x, c.dx, c.nx, ix, s.wx);
+    const int u0 = wrap_index(ix[0] - w.x0, c.nx);
+    if (u0 + 2 >= w.WX) return false;
+    s.skn = s.skh = 0;
+    if constexpr (YF == 1) {
+        tsc_periodic(y, c.dy, c.ny, jn, s.wn);
+        const int v0 = wrap_index(jn[0] - w.y0, c.ny);
+        if (v0 + 2 >= w.WY) return false;
+        s.kn = s.kh = v0 * w.WX + u0;
+    } else {
+        tsc_freehand_w(c.yax, w, y, jn, s.wn, jh, s.wh);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            if (jn[j] < 0 || jn[j] >= c.ny) s.skn |= 1u << j;
+            else if (jn[j] < w.y0 || jn[j] >= w.y0 + w.WY) return false;
+            if (jh[j] < 0 || jh[j] >= c.ny) s.skh |= 1u << j;
+            else if (jh[j] < w.y0 || jh[j] >= w.y0 + w.WY) return false;
+        }
+        s.kn = (jn[0] - w.y0) * w.WX + u0;
+        s.kh = (jh[0] - w.y0) * w.WX + u0;
+    }
+    return true;
+}
+// The sums of a stencil, g q(fl) + f q(fl+1) per node with the weights and in the order of gather(), so that the
+// values are those of a gather from F.  TWO: also E at two further points in zeta (g1, f1 and g0, f0) from the same
+// reads
+template <int YF, bool TWO>
+__device__ __forceinline__ void win_sums(const Win& w, const WinStencil& s, double g, double f, double E[3], double B[3],
+                                         double g1, double f1, double g0, double f0, double E1[3], double E0[3]) {
+    double v[6] = {0, 0, 0, 0, 0, 0}, a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        if (YF == 1 || !(s.skn >> j & 1u)) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const G3D_LDS f4v* q = w.fld + 3 * (s.kn + j * w.WX + i);
+                const double wt = s.wx[i] * s.wn[j];
+                const f4v p = q[0];
+                const f2v r = *(const G3D_LDS f2v*)(q + 1);
+                const double x0 = p.x, z0 = p.y, x1 = p.w, z1 = r.x;
+                v[0] += wt * (g * x0 + f * x1);
+                v[2] += wt * (g * z0 + f * z1);
+                v[4] += wt * (g * double(p.z) + f * double(r.y));
+                if (TWO) {
+                    a[0] += wt * (g1 * x0 + f1 * x1); a[2] += wt * (g1 * z0 + f1 * z1);
+                    b[0] += wt * (g0 * x0 + f0 * x1); b[2] += wt * (g0 * z0 + f0 * z1);
+                }
+            }
+        }
+        if (YF == 1 || !(s.skh >> j & 1u)) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const G3D_LDS f4v* q = w.fld + 3 * (s.kh + j * w.WX + i);
+                const double wt = s.wx[i] * (YF == 1 ? s.wn[j] : s.wh[j]);
+                const f2v r = *((const G3D_LDS f2v*)(q + 1) + 1);
+                const f4v p = q[2];
+                const double y0 = r.x, y1 = p.y;
+                v[1] += wt * (g * y0 + f * y1);
+                v[3] += wt * (g * double(r.y) + f * double(p.z));
+                v[5] += wt * (g * double(p.x) + f * double(p.w));
+                if (TWO) { a[1] += wt * (g1 * y0 + f1 * y1); b[1] += wt * (g0 * y0 + f0 * y1); }
+            }
+        }
+    }
+    E[0] = v[0]; E[1] = v[1]; E[2] = v[2]; B[0] = v[3]; B[1] = v[4]; B[2] = v[5];
+    if (TWO)
+        for (int k = 0; k < 3; ++k) { E1[k] = a[k]; E0[k] = b[k]; }
+}
+// the factors of slices fl and fl+1 at zeta; false when the pair is not the window's.  A point on slice fl+1 itself
+// (the pair fl+1, fl+2 with f = 0) is 0 q(fl) + 1 q(fl+1): the same sum for finite fields
+__device__ __forceinline__ bool win_pair(const FieldView& c, const Win& w, double zeta, double& g, double& f) {
+    int n; double fz;
+    c.zax.locate(zeta, n, fz);
+    if (n == c.a - 1 && fz > 1 - 1e-9) { n = c.a; fz = 0; }
+    g = 1 - fz; f = fz;
+    if (n - c.a == w.fl) return true;
+    if (n - c.a == w.fl + 1 && fz == 0) { g = 0; f = 1; return true; }
+    return false;
+}
+
+// E, B from the tile's field window: false when the stencil or the slice pair is not in the window (then the caller
 // gathers from F)
+template <int YF>
 __device__ __forceinline__ bool gather_window(const FieldView& c, const Win& w, double x, double y, double zeta,
                                               double E[3], double B[3]) {
     if (!c.self) return false;
-    int n; double fz;
-    c.zax.locate(zeta, n, fz);
-    if (n == c.a - 1 && fz > 1 - 1e-9) { n = c.a; fz = 0; }
-    if (n - c.a != w.fl) return false;
-    int ix[3], jn[3]; double wx[3], wn[3];
-    tsc_periodic(x, c.dx, c.nx, ix, wx);
-    tsc_periodic(y, c.dy, c.ny, jn, wn);
-    const int u0 = wrap_index(ix[0] - w.x0, c.nx), v0 = wrap_index(jn[0] - w.y0, c.ny);
-    if (u0 + 2 >= w.WX || v0 + 2 >= w.WY) return false;
-    const double gz = 1 - fz;
-    int k[9]; double wt[9];
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int i = 0; i < 3; ++i) { k[3 * j + i] = (v0 + j) * w.WX + u0 + i; wt[3 * j + i] = wx[i] * wn[j]; }
-    const int pl = w.WX * w.WY;
-    double v[6];
-#pragma unroll
-    for (int comp = 0; comp < 6; ++comp) {
-        const float* q0 = w.fld + comp * pl;
-        const float* q1 = w.fld + (6 + comp) * pl;
-        double s = 0;
-#pragma unroll
-        for (int t = 0; t < 9; ++t) s += wt[t] * (gz * double(q0[k[t]]) + fz * double(q1[k[t]]));
-        v[comp] = s;
-    }
-    E[0] = v[0]; E[1] = v[1]; E[2] = v[2]; B[0] = v[3]; B[1] = v[4]; B[2] = v[5];
-    return true;
-}
-
-// E, B from the tile's field window on the free-hand y grid (window rows y0 .. y0+WY-1 are node indices; the
-// half-nodes share them): the rows beyond the walls skipped and the same weights and order of the sums as
-// gather_t<0>, so the values are identical; false when a row or column of the stencil or the slice pair is not in
-// the window (then the caller gathers from F)
-__device__ __forceinline__ bool gather_window_fh(const FieldView& c, const Win& w, double x, double y, double zeta,
-                                                 double E[3], double B[3]) {
-    if (!c.self) return false;
-    int n; double fz;
-    c.zax.locate(zeta, n, fz);
-    if (n == c.a - 1 && fz > 1 - 1e-9) { n = c.a; fz = 0; }
-    if (n - c.a != w.fl) return false;
-    int ix[3], jn[3], jh[3]; double wx[3], wn[3], wh[3];
-    tsc_periodic(x, c.dx, c.nx, ix, wx);
-    const int u0 = wrap_index(ix[0] - w.x0, c.nx);
-    if (u0 + 2 >= w.WX) return false;
-    tsc_freehand(c.yax, y, jn, wn, jh, wh);
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-        if (jn[j] >= 0 && jn[j] < c.ny && (jn[j] < w.y0 || jn[j] >= w.y0 + w.WY)) return false;
-        if (jh[j] >= 0 && jh[j] < c.ny && (jh[j] < w.y0 || jh[j] >= w.y0 + w.WY)) return false;
-    }
-    const double gz = 1 - fz;
-    const int pl = w.WX * w.WY;
-#pragma unroll
-    for (int comp = 0; comp < 6; ++comp) {
-        const float* q0 = w.fld + comp * pl;
-        const float* q1 = w.fld + (6 + comp) * pl;
-        const bool hf = half_comp(comp);
-        double v = 0;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            const int jj = hf ? jh[j] : jn[j];
-            const double wy = hf ? wh[j] : wn[j];
-            if (jj < 0 || jj >= c.ny) continue;
-            const int r = (jj - w.y0) * w.WX + u0;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) v += wx[i] * wy * (gz * double(q0[r + i]) + fz * double(q1[r + i]));
-        }
-        if (comp < 3) E[comp] = v; else B[comp - 3] = v;
-    }
+    double g, f;
+    WinStencil s;
+    if (!win_pair(c, w, zeta, g, f) || !win_stencil<YF>(c, w, x, y, s)) return false;
+    win_sums<YF, false>(w, s, g, f, E, B, 0, 0, 0, 0, nullptr, nullptr);
     return true;
 }
 
@@ -106,14 +175,14 @@ __device__ __forceinline__ bool gather_window_fh(const FieldView& c, const Win& 
 struct St { double x, y, zeta, px, py, pz; };
 
 // E, B at a beam particle: from the field window of its workgroup when the stencil and the slice pair lie in it (the
-// same values: gather_window sums as gather does), else from F
-__device__ __forceinline__ bool rhs(const PushArgs& c, const Win* win, const St& Y, double z, double qm, St& d) {
+// same values: the window's sums are gather's), else from F
+__device__ __forceinline__ bool rhs(const PushArgs& c, const Win& win, const St& Y, double z, double qm, St& d) {
     const double g = sqrt(1 + Y.px * Y.px + Y.py * Y.py + Y.pz * Y.pz);
     if (Y.pz < 0.3 * g) return false;
     const double gm = (1 + Y.px * Y.px + Y.py * Y.py) / (g + Y.pz);
     double E[3], B[3], Ee[3], Be[3];
     const double xw = wrap_mod(Y.x, c.fv.Lx), yw = c.fv.yf ? wrap_mod(Y.y, c.fv.Ly) : Y.y;
-    if (!(win && gather_window(c.fv, *win, xw, yw, Y.zeta, E, B))) gather(c.fv, xw, yw, Y.zeta, E, B);
+    if (!(win.WX && gather_window<1>(c.fv, win, xw, yw, Y.zeta, E, B))) gather(c.fv, xw, yw, Y.zeta, E, B);
     c.laser.field(Y.x + c.X0, z, z - (Y.zeta - c.zc), Ee, Be);
     for (int k = 0; k < 3; ++k) { E[k] += Ee[k]; B[k] += Be[k]; }
     const double ip = 1 / Y.pz;
@@ -128,7 +197,7 @@ __device__ __forceinline__ St axpy(const St& a, double h, const St& b) {
 }
 
 // beam particle ip from s0 (or from its hand-over point) to s1 (src/sim_kernels.hpp:98-149)
-__device__ __forceinline__ void push_beam_one(const PushArgs& c, const Win* win, Parts P, long ip, double z0) {
+__device__ __forceinline__ void push_beam_one(const PushArgs& c, const Win& win, Parts P, long ip, double z0) {
     const int alive = P.alive[ip];
     if (alive != 1 && alive != 3) return;
     double z = alive == 3 ? c.s1 - P.rem[ip] : z0;
@@ -156,20 +225,23 @@ __device__ __forceinline__ void push_beam_one(const PushArgs& c, const Win* win,
             const double lim = c.push_phase * Y.pz / (c.laser.kL * (hl > 1e-12 ? hl : 1e-12));
             if (lim < ds) ds = (c.s1 - z) / ceil((c.s1 - z) / lim);
         }
-        St k1, k2, k3, k4;
+        // the four stages as a loop (one copy of the gather in the code; unrolled they took 255 VGPRs and 100 KB of
+        // instructions: 106 us against 115 for 2^18 electrons), the sums k1 + 2 k2 + 2 k3 + k4 from the left
+        St k{}, A{};
         const double hd = 0.5 * ds;
-        if (!(rhs(c, win, Y, z, qm, k1) && rhs(c, win, axpy(Y, hd, k1), z + hd, qm, k2) &&
-              rhs(c, win, axpy(Y, hd, k2), z + hd, qm, k3) && rhs(c, win, axpy(Y, ds, k3), z + ds, qm, k4))) {
-            P.alive[ip] = 0;
-            return;
+#pragma unroll 1
+        for (int st = 0; st < 4; ++st) {
+            const double hs = st == 0 ? 0.0 : (st == 3 ? ds : hd);
+            const St Ys = st == 0 ? Y : axpy(Y, hs, k);
+            if (!rhs(c, win, Ys, z + hs, qm, k)) { P.alive[ip] = 0; return; }
+            if (st == 0) A = k;
+            else {
+                const double m = st == 3 ? 1.0 : 2.0;
+                A = St{A.x + m * k.x, A.y + m * k.y, A.zeta + m * k.zeta, A.px + m * k.px, A.py + m * k.py, A.pz + m * k.pz};
+            }
         }
         const double w = ds / 6;
-        Y.x += w * (k1.x + 2 * k2.x + 2 * k3.x + k4.x);
-        Y.y += w * (k1.y + 2 * k2.y + 2 * k3.y + k4.y);
-        Y.zeta += w * (k1.zeta + 2 * k2.zeta + 2 * k3.zeta + k4.zeta);
-        Y.px += w * (k1.px + 2 * k2.px + 2 * k3.px + k4.px);
-        Y.py += w * (k1.py + 2 * k2.py + 2 * k3.py + k4.py);
-        Y.pz += w * (k1.pz + 2 * k2.pz + 2 * k3.pz + k4.pz);
+        Y.x += w * A.x; Y.y += w * A.y; Y.zeta += w * A.zeta; Y.px += w * A.px; Y.py += w * A.py; Y.pz += w * A.pz;
         z += ds;
     }
     store(Y);
@@ -182,7 +254,7 @@ __device__ __forceinline__ void push_beam_one(const PushArgs& c, const Win* win,
 __global__ void __launch_bounds__(kT) k_bunch_push(PushArgs c, Parts P, long np, double z0) {
     const long ip = long(blockIdx.x) * blockDim.x + threadIdx.x;
     if (ip >= np) return;
-    push_beam_one(c, nullptr, P, ip, z0);
+    push_beam_one(c, Win{}, P, ip, z0);
 }
 
 // ---- the beam push with field windows (Fourier y): the particles binned by (slice pair, transverse tile of kBT x kBT
@@ -237,40 +309,34 @@ __global__ void __launch_bounds__(kT) k_bpush_chunks(const unsigned long long* k
 __global__ void __launch_bounds__(kT) k_bunch_push_win(PushArgs c, Parts P, const unsigned long long* key,
                                                        const unsigned* idx, const long* chunk, const int* nchunk,
                                                        int cap, int ntx, int nty, long nbin, double z0) {
-    __shared__ float win[12 * kBW * kBW];
+    __shared__ f4v win[3 * kBW * kBW];
     const FieldView& F = c.fv;
     const int nc = min(*nchunk, cap);
     for (int q = blockIdx.x; q < nc; q += gridDim.x) {
         const long lo = chunk[2 * q], hi = chunk[2 * q + 1];
         const unsigned long long k = key[lo];
-        if (k == (unsigned long long)nbin) {         // outside the slices of F: no window
-            for (long t = lo + threadIdx.x; t < hi; t += blockDim.x) push_beam_one(c, nullptr, P, long(idx[t]), z0);
-            continue;
-        }
         const int tx = int(k % (unsigned long long)ntx), ty = int((k / ntx) % (unsigned long long)nty);
         const int fl = int(k / ((unsigned long long)ntx * nty));
         const int x0 = tx * kBT - 1 - kBM, y0 = ty * kBT - 1 - kBM;
         constexpr int pl = kBW * kBW;
         const long cs = long(F.ns + 2) * F.nk;
+        const bool none = k == (unsigned long long)nbin;   // outside the slices of F: no window (WX = 0)
         __syncthreads();                             // the previous chunk's particles are done with the window
-        for (int r = threadIdx.x; r < pl; r += blockDim.x) {
+        for (int r = none ? pl : threadIdx.x; r < pl; r += blockDim.x) {
             const int v = r / kBW, u = r - v * kBW;
             const float* src = F.F + long(fl) * F.nk + long(wrap_index(y0 + v, F.ny)) * F.nx + wrap_index(x0 + u, F.nx);
-#pragma unroll
-            for (int comp = 0; comp < 6; ++comp) {
-                win[comp * pl + r] = src[comp * cs];
-                win[(6 + comp) * pl + r] = src[comp * cs + F.nk];
-            }
+            win_node((G3D_LDS f4v*)win + 3 * r, src, cs, F.nk, true);
         }
         __syncthreads();
-        const Win w{nullptr, win, x0, y0, kBW, kBW, fl};
-        for (long t = lo + threadIdx.x; t < hi; t += blockDim.x) push_beam_one(c, &w, P, long(idx[t]), z0);
+        const Win w{nullptr, (const G3D_LDS f4v*)win, nullptr, x0, y0, none ? 0 : kBW, kBW, fl, 0, 0};
+        for (long t = lo + threadIdx.x; t < hi; t += blockDim.x) push_beam_one(c, w, P, long(idx[t]), z0);
     }
 }
 
 // TSC deposit of f (dt/Delta) v/(h dx dy) (src/sim_stream.hpp:33-64) into plane comp of the half-cell current:
 // the tile's LDS window when the whole 3 x 3 stencil lies inside it, else jsr with global atomics.  Zero
-// contributions are skipped (adding +-0 to a sum that starts at +0 never changes it).
+// contributions are skipped (adding +-0 to a sum that starts at +0 never changes it).  The charge density planes
+// only when rho: their one reader, the density lines, takes the last pass of a half-cell.
 // a deposit into the current planes: float atomics in the FP32-mixed form (c.Jf), else FP64
 __device__ __forceinline__ void jadd(const StreamArgs& c, long k, double v) {
     if (c.Jf) atomicAdd(&c.Jf[k], float(v));
@@ -278,8 +344,8 @@ __device__ __forceinline__ void jadd(const StreamArgs& c, long k, double v) {
 }
 
 template <int YF>
-__device__ __forceinline__ void sdeposit(const StreamArgs& c, const Win* win, double x, double y, double f, double vx,
-                                         double vy, double vz) {
+__device__ __forceinline__ void sdeposit(const StreamArgs& c, const Win& win, double x, double y, double f, double vx,
+                                         double vy, double vz, bool rho) {
     const FieldView& P = c.fv;
     int ix[3], jn[3], jh[3]; double wx[3], wn[3], wh[3];
     tsc_periodic(x, P.dx, P.nx, ix, wx);
@@ -295,25 +361,25 @@ __device__ __forceinline__ void sdeposit(const StreamArgs& c, const Win* win, do
             for (int u = 0; u < 3; ++u) w[3 * v + u] = f * wx[u] * wn[v] * c.ia[0];
         int u0 = 0, v0 = 0;
         bool in = false;
-        if (win) {
-            u0 = wrap_index(ix[0] - win->x0, P.nx);
-            v0 = wrap_index(jn[0] - win->y0, P.ny);
-            in = u0 + 2 < win->WX && v0 + 2 < win->WY;
+        if (win.WX) {
+            u0 = wrap_index(ix[0] - win.x0, P.nx);
+            v0 = wrap_index(jn[0] - win.y0, P.ny);
+            in = u0 + 2 < win.WX && v0 + 2 < win.WY;
         }
         if (in) {
-            const long wpl = long(win->WX) * win->WY;
+            const long wpl = long(win.WX) * win.WY;
 #pragma unroll
             for (int v = 0; v < 3; ++v)
 #pragma unroll
                 for (int u = 0; u < 3; ++u) {
-                    double* L = win->lds + long(v0 + v) * win->WX + (u0 + u);
+                    const ldsd L = win.lds + long(v0 + v) * win.WX + (u0 + u);
                     const double ww = w[3 * v + u];
                     if (mv) {
-                        atomicAdd(L, ww * vx);
-                        atomicAdd(L + wpl, ww * vy);
-                        atomicAdd(L + 2 * wpl, ww * vz);
+                        lds_add(L, ww * vx);
+                        lds_add(L + wpl, ww * vy);
+                        lds_add(L + 2 * wpl, ww * vz);
                     }
-                    atomicAdd(L + cq * wpl, ww);
+                    if (rho) lds_add(L + cq * wpl, ww);
                 }
             return;
         }
@@ -328,42 +394,46 @@ __device__ __forceinline__ void sdeposit(const StreamArgs& c, const Win* win, do
                     jadd(c, nk + k, ww * vy);
                     jadd(c, 2 * nk + k, ww * vz);
                 }
-                jadd(c, cq * nk + k, ww);
+                if (rho) jadd(c, cq * nk + k, ww);
             }
         return;
     }
-    tsc_freehand(P.yax, y, jn, wn, jh, wh);
-    if (win) {
+    tsc_freehand_w(P.yax, win, y, jn, wn, jh, wh);
+    if (win.WX) {
         // the window's rows are node (and half-node) indices from y0, not wrapped: the walls bound the grid
-        const int u0 = wrap_index(ix[0] - win->x0, P.nx), vn = jn[0] - win->y0, vh = jh[0] - win->y0;
-        if (u0 + 2 < win->WX && vn >= 0 && vn + 2 < win->WY && vh >= 0 && vh + 2 < win->WY) {
-            const long wpl = long(win->WX) * win->WY;
+        const int u0 = wrap_index(ix[0] - win.x0, P.nx), vn = jn[0] - win.y0, vh = jh[0] - win.y0;
+        if (u0 + 2 < win.WX && vn >= 0 && vn + 2 < win.WY && vh >= 0 && vh + 2 < win.WY) {
+            const long wpl = long(win.WX) * win.WY;
+#pragma unroll
             for (int v = 0; v < 3; ++v) {
                 const bool nod = jn[v] >= 1 && jn[v] <= P.ny - 1, hal = jh[v] >= 0 && jh[v] <= P.ny - 1;
+#pragma unroll
                 for (int u = 0; u < 3; ++u) {
                     if (nod) {
-                        double* L = win->lds + long(vn + v) * win->WX + (u0 + u);
+                        const ldsd L = win.lds + long(vn + v) * win.WX + (u0 + u);
                         const double w = f * wx[u] * wn[v] * c.ia[jn[v]];
-                        if (mv) { atomicAdd(L, w * vx); atomicAdd(L + 2 * wpl, w * vz); }
-                        atomicAdd(L + cq * wpl, w);
+                        if (mv) { lds_add(L, w * vx); lds_add(L + 2 * wpl, w * vz); }
+                        if (rho) lds_add(L + cq * wpl, w);
                     }
                     if (hal && mv) {
-                        double* L = win->lds + long(vh + v) * win->WX + (u0 + u);
-                        atomicAdd(L + wpl, f * wx[u] * wh[v] * c.id[jh[v]] * vy);
+                        const ldsd L = win.lds + long(vh + v) * win.WX + (u0 + u);
+                        lds_add(L + wpl, f * wx[u] * wh[v] * c.id[jh[v]] * vy);
                     }
                 }
             }
             return;
         }
     }
+#pragma unroll
     for (int v = 0; v < 3; ++v) {
         const bool nod = jn[v] >= 1 && jn[v] <= P.ny - 1, hal = jh[v] >= 0 && jh[v] <= P.ny - 1;
+#pragma unroll
         for (int u = 0; u < 3; ++u) {
             if (nod) {
                 const long k = long(jn[v]) * P.nx + ix[u];
                 const double w = f * wx[u] * wn[v] * c.ia[jn[v]];
                 if (mv) { jadd(c, k, w * vx); jadd(c, 2 * nk + k, w * vz); }
-                jadd(c, cq * nk + k, w);
+                if (rho) jadd(c, cq * nk + k, w);
             }
             if (hal && mv) {
                 const long k = long(jh[v]) * P.nx + ix[u];
@@ -374,26 +444,39 @@ __device__ __forceinline__ void sdeposit(const StreamArgs& c, const Win* win, do
 }
 
 // E, B at (x, y, zeta) (x, y wrapped as the grid wants): from the tile's field window when it holds the stencil,
-// else from F; the values are the same either way
-template <int YF>
-__device__ __forceinline__ void gather_stream(const FieldView& P, const Win* win, double x, double y, double zeta,
-                                              double E[3], double B[3]) {
-    bool got = false;
-    if (win && win->fld) {
-        if constexpr (YF == 1) got = gather_window(P, *win, x, y, zeta, E, B);
-        else got = gather_window_fh(P, *win, x, y, zeta, E, B);
+// else from F; the values are the same either way.  two: also E at zeta1 and zeta0 (the ends of an ion's path, where
+// the ionization rate is taken), from the same stencil
+template <int YF, bool TWO>
+__device__ __forceinline__ void gather_stream(const FieldView& P, const Win& win, double x, double y, double zeta,
+                                              double E[3], double B[3], bool two, double zeta1, double zeta0,
+                                              double E1[3], double E0[3]) {
+    if (win.fld) {
+        double g, f, g1 = 0, f1 = 0, g0 = 0, f0 = 0;
+        WinStencil s;
+        bool got = win_pair(P, win, zeta, g, f);
+        if (TWO && two) got = got && win_pair(P, win, zeta1, g1, f1) && win_pair(P, win, zeta0, g0, f0);
+        if (got && win_stencil<YF>(P, win, x, y, s)) {
+            if (TWO && two) win_sums<YF, true>(win, s, g, f, E, B, g1, f1, g0, f0, E1, E0);
+            else win_sums<YF, false>(win, s, g, f, E, B, 0, 0, 0, 0, nullptr, nullptr);
+            return;
+        }
     }
-    if (!got) gather_t<YF>(P, x, y, zeta, E, B);
+    if (TWO && two) {
+        double D[3];
+        gather_t<YF>(P, x, y, zeta1, E1, D);
+        gather_t<YF>(P, x, y, zeta0, E0, D);
+    }
+    gather_t<YF>(P, x, y, zeta, E, B);
 }
 
-// |E| of the grid and the analytic laser (src/sim_stream.hpp:67-74)
-template <int YF>
-__device__ __forceinline__ double field_abs(const StreamArgs& c, const Win* win, double x, double y, double z,
-                                            double zeta) {
-    double E[3], B[3], Ee[3], Be[3];
-    gather_stream<YF>(c.fv, win, wrap_mod(x, c.fv.Lx), YF ? wrap_mod(y, c.fv.Ly) : y, zeta, E, B);
-    c.laser.field(x + c.X0, z, z - (zeta - c.zc), Ee, Be);
-    for (int k = 0; k < 3; ++k) E[k] += Ee[k];
+// |E| of the grid (E) and the analytic laser (src/sim_stream.hpp:67-74)
+template <bool LASER>
+__device__ __forceinline__ double field_abs(const StreamArgs& c, double x, double z, double zeta, double E[3]) {
+    if (LASER) {
+        double Ee[3], Be[3];
+        c.laser.field(x + c.X0, z, z - (zeta - c.zc), Ee, Be);
+        for (int k = 0; k < 3; ++k) E[k] += Ee[k];
+    }
     return sqrt(E[0] * E[0] + E[1] * E[1] + E[2] * E[2]);
 }
 
@@ -435,7 +518,7 @@ __device__ __forceinline__ void ionize(const StreamArgs& c, PState& p, double E1
 // YF: the grid (1 Fourier y, 0 free-hand y); ION: the list may hold ions; LASER: the deck has the analytic laser
 // (without it the laser's field is zero and its evaluation would only cost registers)
 template <int YF, bool ION, bool LASER>
-__device__ __forceinline__ void stream_one(const StreamArgs& c, const Win* win, PState& p) {
+__device__ __forceinline__ void stream_one(const StreamArgs& c, const Win& win, PState& p) {
     const int n = c.n;
     const double zn = c.zs[n], zn1 = c.zs[n + 1], h = zn1 - zn;
     if (p.alive == 6) {
@@ -446,24 +529,38 @@ __device__ __forceinline__ void stream_one(const StreamArgs& c, const Win* win, 
     const double hl = p.zeta >= zn1 - 1e-9 * h ? h : (p.zeta - zn > 0 ? p.zeta - zn : 0.0);
     const FieldView& P = c.fv;
     const bool ion = ION && is_ion(p.sp);
-    if (ion && !c.ions[p.sp - SP_ION].mobile) {
-        const double f = p.q * p.w * hl / (c.Delta * h * P.dx);
-        if (f != 0) sdeposit<YF>(c, win, p.x, p.y, f, 0, 0, 0);
-        const double E1 = field_abs<YF>(c, win, p.x, p.y, p.z, p.zeta), E0 = field_abs<YF>(c, win, p.x, p.y, p.z, zn);
-        p.zeta = zn;
-        ionize(c, p, E1, E0, hl);
-        return;
-    }
+    const bool ionizing = ion && c.ions[p.sp - SP_ION].ionizing, fixed = ion && !c.ions[p.sp - SP_ION].mobile;
+    const bool rho = !c.skip_state;
+    double E1a = 0, E0a = 0;             // |E| at the ends of the path of an ionizing ion
+    double E[3], B[3];
     const double zeta0 = p.zeta;
     const double g0 = sqrt(1 + p.px * p.px + p.py * p.py + p.pz * p.pz);
     const double omv0 = (1 + p.px * p.px + p.py * p.py) / (g0 * (g0 + p.pz));
     const double dt0 = hl / omv0;
-    const double xm = p.x + 0.5 * dt0 * p.px / g0, ym = p.y + 0.5 * dt0 * p.py / g0;
-    const double zm = p.z + 0.5 * dt0 * p.pz / g0, zetam = p.zeta - 0.5 * hl;
-    double E[3], B[3], Ee[3], Be[3];
-    const double xg = wrap_mod(xm, P.Lx), yg = YF ? wrap_mod(ym, P.Ly) : ym;
-    gather_stream<YF>(P, win, xg, yg, zetam, E, B);
+    double xm = p.x, ym = p.y, zm = p.z;
+    if (!fixed) {
+        xm = p.x + 0.5 * dt0 * p.px / g0; ym = p.y + 0.5 * dt0 * p.py / g0;
+        zm = p.z + 0.5 * dt0 * p.pz / g0;
+    }
+    const double zetam = p.zeta - 0.5 * hl;
+    {
+        double E1[3], E0[3];
+        const double xg = wrap_mod(xm, P.Lx), yg = YF ? wrap_mod(ym, P.Ly) : ym;
+        gather_stream<YF, ION>(P, win, xg, yg, zetam, E, B, ionizing, zeta0, zn, E1, E0);
+        if (ION && ionizing) {
+            E1a = field_abs<LASER>(c, xm, zm, zeta0, E1);
+            E0a = field_abs<LASER>(c, xm, zm, zn, E0);
+        }
+    }
+    if (fixed) {
+        const double f = p.q * p.w * hl / (c.Delta * h * P.dx);
+        if (f != 0) sdeposit<YF>(c, win, p.x, p.y, f, 0, 0, 0, rho);
+        p.zeta = zn;
+        if (ionizing) ionize(c, p, E1a, E0a, hl);
+        return;
+    }
     if (LASER) {
+        double Ee[3], Be[3];
         c.laser.field(xm + c.X0, zm, zm - (zetam - c.zc), Ee, Be);
         for (int k = 0; k < 3; ++k) { E[k] += Ee[k]; B[k] += Be[k]; }
     }
@@ -493,16 +590,22 @@ __device__ __forceinline__ void stream_one(const StreamArgs& c, const Win* win, 
     p.z = trapped ? c.s1 : p.z + vz * dt;
     p.px = ux; p.py = uy; p.pz = uz;
     p.zeta = zeta_end;
-    const double f = p.q * p.w * dt / (c.Delta * h * P.dx);
-    if (f != 0) sdeposit<YF>(c, win, 0.5 * (xo + p.x), 0.5 * (yo + p.y), f, vx, vy, vz);
-    if (!YF && (p.y < c.ylo || p.y > c.yhi)) { p.alive = 0; return; }
-    if (ion && !trapped && c.ions[p.sp - SP_ION].ionizing)
-        ionize(c, p, field_abs<YF>(c, win, xm, ym, zm, zeta0), field_abs<YF>(c, win, xm, ym, zm, zn), dt);
-    if (trapped) {
-        p.alive = 5;
-        const double vze = uz / g1;
-        if (vze >= c.vz_beam) sdeposit<YF>(c, win, p.x, p.y, p.q * p.w / (h * P.dx * vze), ux / g1, uy / g1, vze);
+    const bool out = !YF && (p.y < c.ylo || p.y > c.yhi);
+    // the streaming current, then for a trapped particle that joins the beam its beam current (one copy of the
+    // deposit in the code)
+    double f = p.q * p.w * dt / (c.Delta * h * P.dx);
+    double xd = 0.5 * (xo + p.x), yd = 0.5 * (yo + p.y);
+    const double vze = uz / g1;
+    const bool join = trapped && !out && vze >= c.vz_beam;
+#pragma unroll 1
+    for (int d = 0;; ++d) {
+        if (f != 0 || d) sdeposit<YF>(c, win, xd, yd, f, vx, vy, vz, rho);
+        if (d || !join) break;
+        xd = p.x; yd = p.y; f = p.q * p.w / (h * P.dx * vze); vx = ux / g1; vy = uy / g1; vz = vze;
     }
+    if (out) { p.alive = 0; return; }
+    if (ION && ionizing && !trapped) ionize(c, p, E1a, E0a, dt);
+    if (trapped) p.alive = 5;
 }
 
 __device__ __forceinline__ PState load_pstate(const Parts& S, long i) {
@@ -512,99 +615,99 @@ __device__ __forceinline__ PState load_pstate(const Parts& S, long i) {
 
 // p: the state of list entry i (loaded by the caller); the pushed state goes to D[i]
 template <int YF, bool ION, bool LASER>
-__device__ __forceinline__ void stream_index(const StreamArgs& c, const Win* win, PState p, Parts D, long i) {
+__device__ __forceinline__ void stream_index(const StreamArgs& c, const Win& win, PState p, Parts D, long i) {
     stream_one<YF, ION, LASER>(c, win, p);
     if (c.skip_state) return;
     D.x[i] = p.x; D.y[i] = p.y; D.zeta[i] = p.zeta; D.px[i] = p.px; D.py[i] = p.py; D.pz[i] = p.pz;
     D.z[i] = p.z; D.q[i] = p.q; D.qm[i] = p.qm; D.alive[i] = p.alive;
 }
 
+// waves per SIMD that the register allocation of an instance must allow (0: the compiler's choice): 4 for the plain
+// electron kernel (28 us at 256 x 256 against 31 with 3); the others spill too much for a cap (free-hand y with ions at
+// 512 x 386: 439 us with 2 waves, 528 capped for 4)
+constexpr int stream_waves(int YF, bool ION, bool LASER) { return YF == 1 && !ION && !LASER ? 4 : 1; }
+
 // workgroups 0 .. ntile-1: the particles of one tile with the LDS window, written to the tile's slab at the end;
 // the following workgroups: the untiled particles from off[ntile] on, one per lane, global atomics
 template <int YF, bool ION, bool LASER>
-__global__ void __launch_bounds__(kStreamBlockMax) k_stream_halfcell(StreamArgs c, Parts S, Parts D, long n,
+__global__ void __launch_bounds__(kStreamBlockMax)
+__attribute__((amdgpu_waves_per_eu(stream_waves(YF, ION, LASER)))) k_stream_halfcell(StreamArgs c, Parts S, Parts D, long n,
                                                                      TileGeom tg) {
-    extern __shared__ double win_lds[];
+    extern __shared__ __align__(16) double win_lds[];
     const long b = blockIdx.x;
-    if (b < tg.ntile) {
-        // free-hand y (every gather reads F): the tiles of one XCD a band of consecutive tile rows, so that
-        // neighbouring tiles meet in one L2 (workgroup b runs on XCD b mod 8)
-        const long t = (tg.fh && (tg.ntile & 7) == 0) ? (b & 7) * (tg.ntile >> 3) + (b >> 3) : b;
-        // the particles binned into this tile (tg.idx: indices into the list; null: the contiguous load ranges).
-        // The range, this lane's first particle and its state first: their dependent loads overlap those of the
-        // field window.
-        const long lo = tg.off[t], hi = tg.off[t + 1];
-        long k = lo + threadIdx.x;
-        long i = k < hi ? (tg.idx ? long(tg.idx[k]) : k) : 0;
-        PState p{};
-        if (k < hi) p = load_pstate(S, i);
-        const int pl = tg.WX * tg.WY;
-        const long wn = 5L * pl;
-        const int tx = int(t % tg.ntx), ty = int(t / tg.ntx);
-        const int x0 = tx * tg.TX - 1 - tg.M, y0 = ty * tg.TY - 1 - tg.M;
-        const FieldView& F = c.fv;
-        const int fl = c.n - F.a;
-        float* fw = reinterpret_cast<float*>(win_lds + wn);
-        for (long r = threadIdx.x; r < wn; r += blockDim.x) win_lds[r] = 0;
+    const bool tiled = b < tg.ntile;
+    // free-hand y (every gather reads F): the tiles of one XCD a band of consecutive tile rows, so that
+    // neighbouring tiles meet in one L2 (workgroup b runs on XCD b mod 8)
+    const long t = (tg.fh && (tg.ntile & 7) == 0) ? (b & 7) * (tg.ntile >> 3) + (b >> 3) : b;
+    // the particles binned into this tile (tg.idx: indices into the list; null: the contiguous load ranges), or a
+    // block of the untiled rest.  The range, this lane's first particle and its state first: their dependent loads
+    // overlap those of the field window.
+    const int* idx = tiled ? tg.idx : nullptr;
+    const long lo = tiled ? tg.off[t] : tg.n_tiled + (b - tg.ntile) * blockDim.x;
+    const long hi = tiled ? tg.off[t + 1] : (lo + blockDim.x < n ? lo + blockDim.x : n);
+    long k = lo + threadIdx.x;
+    long i = k < hi ? (idx ? long(idx[k]) : k) : 0;
+    PState p{};
+    if (k < hi) p = load_pstate(S, i);
+    const int pl = tg.WX * tg.WY;
+    const long wn = 5L * pl;
+    const int tx = int(t % (tiled ? tg.ntx : 1)), ty = tiled ? int(t / tg.ntx) : 0;
+    const int x0 = tx * tg.TX - 1 - tg.M, y0 = ty * tg.TY - 1 - tg.M;
+    const FieldView& F = c.fv;
+    const int fl = c.n - F.a;
+    const ldsd dep = (ldsd)win_lds;
+    Win w{};
+    if (tiled) {
+        G3D_LDS f4v* fw = (G3D_LDS f4v*)(dep + ((wn + 1) & ~1L));
+        for (long r = threadIdx.x; r < wn; r += blockDim.x) dep[r] = 0;
         const bool fwin = tg.fwin && F.self;
-        // slices fl, fl + 1 of the 6 components: [slice][comp][v][u]; one node per lane, 12 loads.  Free-hand y: the
-        // rows beyond the walls are never read (zero)
+        // slices fl, fl + 1 of the 6 components, one node per lane, 12 loads.  Free-hand y: the rows beyond the walls
+        // are never read (zero)
         if (fwin)
             for (int r = threadIdx.x; r < pl; r += blockDim.x) {
                 const int v = r / tg.WX, u = r - v * tg.WX;
                 const int gx = wrap_index(x0 + u, F.nx), gy = YF ? wrap_index(y0 + v, F.ny) : y0 + v;
                 const bool in = YF || (gy >= 0 && gy < F.ny);
                 const float* src = F.F + long(fl) * F.nk + long(in ? gy : 0) * F.nx + gx;
-                const long cs = long(F.ns + 2) * F.nk;
-#pragma unroll
-                for (int comp = 0; comp < 6; ++comp) {
-                    fw[comp * pl + r] = in ? src[comp * cs] : 0.0f;
-                    fw[(6 + comp) * pl + r] = in ? src[comp * cs + F.nk] : 0.0f;
-                }
+                win_node(fw + 3 * r, src, long(F.ns + 2) * F.nk, F.nk, in);
             }
+        w = Win{dep, fwin ? fw : nullptr, nullptr, x0, y0, tg.WX, tg.WY, fl, 0, 0};
+        if (YF == 0 && !F.yax.uniform && F.yax.n >= 3) {         // the y nodes of the window's rows
+            const int nn = F.yax.n;
+            w.y_lo = y0 < 0 ? 0 : (y0 > nn - 2 ? nn - 2 : y0);
+            const int hi_r = y0 + tg.WY > nn - 1 ? nn - 1 : (y0 + tg.WY < w.y_lo + 1 ? w.y_lo + 1 : y0 + tg.WY);
+            w.nyn = hi_r - w.y_lo;
+            const ldsd hx = (ldsd)(fw + (fwin ? 3 * pl : 0));
+            for (int r = threadIdx.x; r <= w.nyn; r += blockDim.x) hx[r] = F.yax.X[w.y_lo + r];
+            w.yn = hx;
+        }
         __syncthreads();
-        Win w{win_lds, fwin ? fw : nullptr, x0, y0, tg.WX, tg.WY, fl};
-        // free-hand y: the y locates of this tile's particles search the window's rows first
-        StreamArgs cl = c;
-        if (YF == 0 && !c.fv.yax.uniform && c.fv.yax.n >= 3) {
-            const int nn = c.fv.yax.n;
-            const int lo_r = y0 < 0 ? 0 : (y0 > nn - 2 ? nn - 2 : y0);
-            const int hi_r = y0 + tg.WY > nn - 1 ? nn - 1 : (y0 + tg.WY < lo_r + 1 ? lo_r + 1 : y0 + tg.WY);
-            cl.fv.yax.hlo = lo_r; cl.fv.yax.hhi = hi_r;
+    }
+    const double zn = c.zs[c.n];
+    unsigned cnt = 0;
+    while (k < hi) {
+        cnt += pushed_through(p.alive, p.zeta, zn);
+        stream_index<YF, ION, LASER>(c, w, p, D, i);
+        k += blockDim.x;
+        if (k < hi) {
+            i = idx ? long(idx[k]) : k;
+            p = load_pstate(S, i);
         }
-        const double zn = c.zs[c.n];
-        unsigned cnt = 0;
-        while (k < hi) {
-            cnt += pushed_through(p.alive, p.zeta, zn);
-            stream_index<YF, ION, LASER>(cl, &w, p, D, i);
-            k += blockDim.x;
-            if (k < hi) {
-                i = tg.idx ? long(tg.idx[k]) : k;
-                p = load_pstate(S, i);
-            }
-        }
+    }
+    if (tiled) {
         __syncthreads();
         if (YF == 1 && !c.Jf) {
             double* sl = tg.slab + t * wn;
-            for (long r = threadIdx.x; r < wn; r += blockDim.x) sl[r] = win_lds[r];
+            for (long r = threadIdx.x; r < wn; r += blockDim.x) sl[r] = dep[r];
         } else                  // into the current planes (free-hand y: rows outside the walls hold nothing)
             for (long r = threadIdx.x; r < wn; r += blockDim.x) {
-                const double v = win_lds[r];
+                const double v = dep[r];
                 if (v == 0) continue;
                 const int cc = int(r / pl), rr = int(r - long(cc) * pl), vv = rr / tg.WX, u = rr - vv * tg.WX;
                 const int gy = YF ? wrap_index(y0 + vv, F.ny) : y0 + vv;
                 if (gy < 0 || gy >= F.ny) continue;
                 jadd(c, cc * F.nk + long(gy) * F.nx + wrap_index(x0 + u, F.nx), v);
             }
-        if (c.npush) add_pushes(c.npush, cnt);
-        return;
-    }
-    const long i = tg.n_tiled + (b - tg.ntile) * blockDim.x + threadIdx.x;
-    unsigned cnt = 0;
-    if (i < n) {
-        const PState p = load_pstate(S, i);
-        cnt = pushed_through(p.alive, p.zeta, c.zs[c.n]);
-        stream_index<YF, ION, LASER>(c, nullptr, p, D, i);
     }
     if (c.npush) add_pushes(c.npush, cnt);
 }
@@ -822,8 +925,12 @@ void stream_halfcell(const StreamArgs& a, Parts src, Parts dst, long nstrm, cons
     const int bs = tg.ntile ? tg.block : kT;
     if (bs < 64 || bs > kStreamBlockMax || bs % 64) throw std::runtime_error("stream half-cell: bad block size");
     const long tail_blocks = nstrm > tg.n_tiled ? long(blocks_for(nstrm - tg.n_tiled, bs)) : 0;
-    // the deposit window (5 double planes) and the field window (12 float planes)
-    const size_t lds = tg.ntile ? size_t(tg.WX) * tg.WY * (5 * sizeof(double) + (tg.fwin ? 12 * sizeof(float) : 0)) : 0;
+    // the deposit window (5 double planes, an even number of values), the field window (12 floats per node) and the
+    // window's y nodes of the free-hand grid
+    const size_t pl = size_t(tg.WX) * tg.WY;
+    const size_t lds = tg.ntile ? ((5 * pl + 1) & ~size_t(1)) * sizeof(double) + (tg.fwin ? pl * 12 * sizeof(float) : 0) +
+                                      (a.fv.yf ? 0 : size_t(tg.WY + 2) * sizeof(double))
+                                : 0;
     const dim3 grid(unsigned(tg.ntile + tail_blocks)), blk(bs);
     if (a.npush && long(grid.x) > a.npush_cap) throw std::runtime_error("stream half-cell: push counter too small");
     const bool ion = a.ions != nullptr;
