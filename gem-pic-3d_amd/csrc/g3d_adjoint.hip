@@ -12,44 +12,99 @@
 #include "g3d_boris_rev.hpp"
 #include "g3d_kernels.hpp"
 #include "g3d_march_adj.hpp"
+#include "g3d_march_half.hpp"
 #include "g3d_runtime.hpp"
 
 namespace g3d {
 namespace {
 
-// slices lo ... hi-1 of every mode, rear to front: the transpose of k_march_all
+// Slices lo ... hi-1 of every mode, rear to front: the transpose of the march.  Like k_march_staged, two lanes per
+// mode (one real half-system each) and 32 modes per workgroup: wave 0 runs the chain from LDS, waves 1-3 load the next
+// block of kAdjB slices (one each) into the other of two buffers and clear L_x, L_y, which are not inputs.  As one
+// lane per mode with complex arithmetic and its loads on the chain it took 742 us for 64 x 64 x 256, now 141 us.
+constexpr int kAdjB = 3, kAdjComp = 11;
 __global__ void __launch_bounds__(256) k_march_adj(AdjView c, int lo, int hi) {
-    const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= c.nk) return;
-    Mode6 carry{};                                  // adjoint of slice n's outputs from slice n-1's use of them
-    cx d0x = mk(0), d0y = mk(0), dkx = mk(0), dky = mk(0), dkz = mk(0);   // half-cell n-1 (plane n - a) so far
-    for (int n = lo; n < hi; ++n) {
-        const long o = long(n - c.a) * c.nk + i;
-        const Mode6 r{c.Rx[o] + carry.Rx, c.Ry[o] + carry.Ry, c.Ez[o] + carry.Ez, c.Bz[o] + carry.Bz,
-                      c.Lx[o] + carry.Lx, c.Ly[o] + carry.Ly};
-        Mode6 old, up;
-        CurAdj J;
-        march_mode_adj(c, i, n, r, old, up, J);
-        c.Rx[o] = old.Rx; c.Ry[o] = old.Ry; c.Ez[o] = old.Ez; c.Bz[o] = old.Bz; c.Lx[o] = old.Lx; c.Ly[o] = old.Ly;
-        // plane n - a is half-cell n-1: the "u" currents of slice n-1 and the "d" currents of slice n
-        c.j0x[o] = c.j0x[o] + d0x + J.j0x_d;
-        c.j0y[o] = c.j0y[o] + d0y + J.j0y_d;
-        c.jkx[o] = c.jkx[o] + dkx + J.jkx_d;
-        c.jky[o] = c.jky[o] + dky + J.jky_d;
-        c.jkz[o] = c.jkz[o] + dkz;
-        d0x = J.j0x_u; d0y = J.j0y_u; dkx = J.jkx_u; dky = J.jky_u; dkz = J.jkz_u;
-        carry = up;
+    __shared__ double stg[2 * kAdjB * kAdjComp * 64], wts[2 * kAdjB * 3];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane & 1;
+    const long i = long(blockIdx.x) * 32 + (lane >> 1);
+    const bool on = i < c.nk;
+    const long ic = on ? i : c.nk - 1, p = 2 * ic + half, e = 2 * ic + 1 - half;
+    const int nblk = (hi - lo + kAdjB - 1) / kAdjB;
+    if (wave > 0) {
+        double r[kAdjComp], w[3];
+        const int s0 = wave - 1;
+        auto load = [&](int b) {
+            const int n = lo + b * kAdjB + s0;
+            if (n >= hi) return;
+            const long o = 2 * long(n - c.a) * c.nk;
+            r[0] = dbl(c.Rx)[o + p]; r[1] = dbl(c.Ry)[o + p]; r[2] = dbl(c.Ez)[o + e]; r[3] = dbl(c.Bz)[o + e];
+            r[4] = dbl(c.Lx)[o + p]; r[5] = dbl(c.Ly)[o + p];
+            r[6] = dbl(c.j0x)[o + p]; r[7] = dbl(c.j0y)[o + p]; r[8] = dbl(c.jkx)[o + p]; r[9] = dbl(c.jky)[o + p];
+            r[10] = dbl(c.jkz)[o + e];
+            w[0] = c.wlo[n]; w[1] = c.whi[n]; w[2] = n < c.N - 1 ? c.hcg[n + 2] : 0.0;
+        };
+        auto write = [&](int b) {
+            const int n = lo + b * kAdjB + s0, s = (b & 1) * kAdjB + s0;
+            if (n >= hi) return;
+#pragma unroll
+            for (int q = 0; q < kAdjComp; ++q) stg[(s * kAdjComp + q) * 64 + lane] = r[q];
+            if (lane < 3) wts[3 * s + lane] = w[lane];
+            if (on) {
+                const long o = 2 * long(n - c.a) * c.nk;
+                dbl(c.Lx)[o + p] = 0; dbl(c.Ly)[o + p] = 0;
+            }
+        };
+        load(0);
+        write(0);
+        if (nblk > 1) load(1);
+        for (int b = 0; b < nblk; ++b) {
+            __syncthreads();
+            if (b + 1 < nblk) write(b + 1);
+            if (b + 2 < nblk) load(b + 2);
+        }
+        return;
     }
-    const long o = long(hi - c.a) * c.nk + i;        // plane hi - a: half-cell hi-1
-    c.j0x[o] = c.j0x[o] + d0x;
-    c.j0y[o] = c.j0y[o] + d0y;
-    c.jkx[o] = c.jkx[o] + dkx;
-    c.jky[o] = c.jky[o] + dky;
-    c.jkz[o] = c.jkz[o] + dkz;
+    const int ixx = int(ic % c.nx), j = int(ic / c.nx);
+    const HalfK k = half_k(half, c.kx[ixx], c.ky[j]);
+    HalfDen dn{};
+    Half6 carry{};                                  // adjoint of slice n's outputs from slice n-1's use of them
+    double d0x = 0, d0y = 0, dkx = 0, dky = 0, dkz = 0;      // half-cell n-1 (plane n - a) so far
+    for (int b = 0; b < nblk; ++b) {
+        __syncthreads();
+        for (int s = 0; s < kAdjB; ++s) {
+            const int n = lo + b * kAdjB + s;
+            if (n >= hi) break;
+            const int sb = (b & 1) * kAdjB + s;
+            const double* q = stg + sb * kAdjComp * 64 + lane;
+            const double wl = wts[3 * sb], wu = wts[3 * sb + 1], h = wts[3 * sb + 2];
+            const Half6 r{q[0] + carry.Rx, q[64] + carry.Ry, q[128] + carry.Ez, q[192] + carry.Bz, q[256] + carry.Lx,
+                          q[320] + carry.Ly};
+            const double c0x = q[384], c0y = q[448], ckx = q[512], cky = q[576], ckz = q[640];
+            const bool front = n == c.N - 1;
+            if (!front) dn.set(k, h, c.D);
+            Half6 old;
+            HalfAdjJ J;
+            half_adjoint(k, dn, c.D, h, wl, wu, front, r, old, carry, J);
+            if (on) {
+                const long o = 2 * long(n - c.a) * c.nk;
+                dbl(c.Rx)[o + p] = old.Rx; dbl(c.Ry)[o + p] = old.Ry; dbl(c.Ez)[o + e] = old.Ez; dbl(c.Bz)[o + e] = old.Bz;
+                // plane n - a is half-cell n-1: the "u" currents of slice n-1 and the "d" currents of slice n
+                dbl(c.j0x)[o + p] = c0x + d0x + J.x_d; dbl(c.j0y)[o + p] = c0y + d0y + J.y_d;
+                dbl(c.jkx)[o + p] = ckx + dkx + J.x_d; dbl(c.jky)[o + p] = cky + dky + J.y_d;
+                dbl(c.jkz)[o + e] = ckz + dkz;
+            }
+            d0x = J.j0x_u; d0y = J.j0y_u; dkx = J.jkx_u; dky = J.jky_u; dkz = J.jkz_u;
+        }
+    }
+    if (!on) return;
+    const long o = 2 * long(hi - c.a) * c.nk;        // plane hi - a: half-cell hi-1
+    dbl(c.j0x)[o + p] += d0x; dbl(c.j0y)[o + p] += d0y; dbl(c.jkx)[o + p] += dkx; dbl(c.jky)[o + p] += dky;
+    dbl(c.jkz)[o + e] += dkz;
     if (c.up && hi < c.N) {
-        const long nk = c.nk;
-        c.up[i] = carry.Rx; c.up[nk + i] = carry.Ry; c.up[2 * nk + i] = carry.Ez;
-        c.up[3 * nk + i] = carry.Bz; c.up[4 * nk + i] = carry.Lx; c.up[5 * nk + i] = carry.Ly;
+        const long pl = 2 * c.nk;
+        double* u = dbl(c.up);
+        u[p] = carry.Rx; u[pl + p] = carry.Ry; u[2 * pl + e] = carry.Ez; u[3 * pl + e] = carry.Bz;
+        u[4 * pl + p] = carry.Lx; u[5 * pl + p] = carry.Ly;
     }
 }
 
@@ -171,7 +226,7 @@ int g3d_march_adjoint(const g3d_march_adj_ctx* m, int lo, int hi) {
         v.j0x = m->j0x; v.j0y = m->j0y; v.jkx = m->jkx; v.jky = m->jky; v.jkz = m->jkz;
         v.kx = m->kx; v.ky = m->ky; v.hcg = m->hcg; v.wlo = m->wlo; v.whi = m->whi;
         v.D = m->D; v.a = m->a; v.N = m->N; v.nx = m->nx; v.nk = m->nk;
-        hipLaunchKernelGGL(g3d::k_march_adj, dim3(g3d::blocks_for(v.nk, 256)), dim3(256), 0, g3d::stream(), v, lo,
+        hipLaunchKernelGGL(g3d::k_march_adj, dim3(g3d::blocks_for(v.nk, 32)), dim3(256), 0, g3d::stream(), v, lo,
                            hi);
         g3d::launch_check("march adjoint");
     });
