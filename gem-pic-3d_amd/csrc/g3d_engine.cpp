@@ -253,29 +253,20 @@ Sim::Sim(const Config& c) : cfg(c) {
     if (cfg.plasma_on) setup_tiles();
 }
 
-// Tiles of TX x TY cells (16 x 8 on large grids) with a margin of M nodes around the TSC reach of the tile; a
-// window of WX = TX + 3 + 2M nodes must fit the period, and a window may reach only the neighbouring tiles.
+// The tiles of the streaming list (tile_shape) with a margin of M nodes around the TSC reach of a tile.
 void Sim::setup_tiles() {
-    auto pick = [](int n, int pref) { for (int t = pref; t >= 8; t >>= 1) if (n % t == 0 && n >= 2 * t) return t; return 0; };
-    int px = 16, py = 8;                      // G3D_TILE=<TX>x<TY> (powers of two from 8) for launch-shape sweeps
+    int px = 0, py = 0;                       // G3D_TILE=<TX>x<TY> (powers of two from 8) for launch-shape sweeps
     if (const char* t = getenv("G3D_TILE")) {
         if (sscanf(t, "%dx%d", &px, &py) != 2 || px < 8 || py < 8)
             throw std::runtime_error("G3D_TILE: expected <TX>x<TY>, both at least 8");
     }
-    // free-hand y: rows of py cells from the first node (the last row may be short), the windows end at the walls
-    const int TX = pick(cfg.nx, px), TY = yf ? pick(cfg.ny, py) : (cfg.ny >= 2 * py ? py : 0);
-    if (!TX || !TY) return;
     // G3D_TILE_MARGIN: nodes of drift a window allows (sweeps); 2 for the FP32-mixed electron kernel (its smaller
     // windows load faster than the few more fallbacks to F cost: 24.1 -> 23.7 us at 256 x 256), else 3
     bool ions = false;
     for (const auto& is : cfg.ions) ions = ions || cfg.loaded(is);
     int M = cfg.mixed && yf && !ions ? 2 : 3;
     if (const char* e = getenv("G3D_TILE_MARGIN")) M = std::max(0, atoi(e));
-    M = std::min({M, TX - 1, TY - 1, (cfg.nx - TX - 3) / 2});
-    if (yf) M = std::min(M, (cfg.ny - TY - 3) / 2);
-    if (M < 0) return;
-    tiles.TX = TX; tiles.TY = TY; tiles.M = M; tiles.WX = TX + 3 + 2 * M; tiles.WY = TY + 3 + 2 * M;
-    tiles.ntx = cfg.nx / TX; tiles.nty = (cfg.ny + TY - 1) / TY; tiles.ntile = long(tiles.ntx) * tiles.nty;
+    if (!tile_shape(tiles, cfg.nx, cfg.ny, yf, M, px, py)) return;
     tiles.fh = !yf;
     tiles.fy = yax;
     tile_off.resize(tiles.ntile + 1);

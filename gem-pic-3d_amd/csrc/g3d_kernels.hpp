@@ -75,6 +75,11 @@ struct TileGeom {
     const int* idx;                   // list indices grouped by tile (null: the list itself is tile-ordered)
     double* slab;
 };
+// the tiles of a grid (TX, TY, M, windows and counts of tg; false: the grid is too small): 16 x 8 cells, and 8 x 8 where
+// those would be fewer than the compute units (FP64 electrons, 2 x 2 per cell: 17.6 -> 15.4 us at 128 x 128; 2 x 1 per
+// cell at 64 x 64 14.6 -> 13.9).  A window of TX + 3 + 2 M nodes must fit the period and reach only the neighbouring
+// tiles.  px, py: the preferred tile (0: the above)
+bool tile_shape(TileGeom& tg, int nx, int ny, bool yf, int M, int px = 0, int py = 0);
 // bin the live particles of the list by their current tile: off[0 .. ntile], idx[0 .. off[ntile]); the state of
 // the other particles (final for the rest of the step) is copied from S to D.  cnt, cur: ntile ints of scratch
 void bin_tiles(Parts S, Parts D, long n, const TileGeom& tg, double dx, double dy, int nx, int ny, int* cnt,

@@ -696,7 +696,7 @@ __attribute__((amdgpu_waves_per_eu(stream_waves(YF, ION, LASER)))) k_stream_half
     }
     if (tiled) {
         __syncthreads();
-        if (YF == 1 && !c.Jf) {
+        if (YF == 1 && !c.Jf && !tg.aflush) {
             double* sl = tg.slab + t * wn;
             for (long r = threadIdx.x; r < wn; r += blockDim.x) sl[r] = dep[r];
         } else                  // into the current planes (free-hand y: rows outside the walls hold nothing)
@@ -922,7 +922,9 @@ void stream_halfcell(const StreamArgs& a, Parts src, Parts dst, long nstrm, cons
                      const LaunchTimer& lt) {
     if (nstrm <= 0) return;
     // tile workgroups of tg.block lanes, then the untiled tail in workgroups of the same size
-    const int bs = tg.ntile ? tg.block : kT;
+    // (a short untiled list in workgroups of one wave, whose few waves then spread over the compute units: a half-cell of
+    // 4 x 10^3 particles and its spectra 31.5 -> 26 us, from 8 x 10^3 on no faster)
+    const int bs = tg.ntile ? tg.block : (nstrm <= 6144 ? 64 : kT);
     if (bs < 64 || bs > kStreamBlockMax || bs % 64) throw std::runtime_error("stream half-cell: bad block size");
     const long tail_blocks = nstrm > tg.n_tiled ? long(blocks_for(nstrm - tg.n_tiled, bs)) : 0;
     // the deposit window (5 double planes, an even number of values), the field window (12 floats per node) and the
@@ -962,6 +964,19 @@ void tile_chunks(const TileGeom& tg, int* xtile, long* xstart, int* xcount) {
     hipLaunchKernelGGL(k_tile_chunks, dim3(1), dim3(1024), 0, stream(), tg.off, tg.ntile, tg.chunk, tg.max_extra,
                        xtile, xstart, xcount);
     launch_check("tile chunks");
+}
+bool tile_shape(TileGeom& tg, int nx, int ny, bool yf, int M, int px, int py) {
+    auto pick = [](int n, int pref) { for (int t = pref; t >= 8; t >>= 1) if (n % t == 0 && n >= 2 * t) return t; return 0; };
+    if (!px || !py) { px = long(nx) * ny < 256L * 16 * 8 && yf ? 8 : 16; py = 8; }
+    // free-hand y: rows of py cells from the first node (the last row may be short), the windows end at the walls
+    const int TX = pick(nx, px), TY = yf ? pick(ny, py) : (ny >= 2 * py ? py : 0);
+    if (!TX || !TY) return false;
+    M = std::min({M, TX - 1, TY - 1, (nx - TX - 3) / 2});
+    if (yf) M = std::min(M, (ny - TY - 3) / 2);
+    if (M < 0) return false;
+    tg.TX = TX; tg.TY = TY; tg.M = M; tg.WX = TX + 3 + 2 * M; tg.WY = TY + 3 + 2 * M;
+    tg.ntx = nx / TX; tg.nty = (ny + TY - 1) / TY; tg.ntile = long(tg.ntx) * tg.nty;
+    return true;
 }
 void bin_tiles(Parts S, Parts D, long n, const TileGeom& tg, double dx, double dy, int nx, int ny, int* cnt,
                int* cur, long* off, int* idx) {
