@@ -804,29 +804,32 @@ void Sim::sponge_and_real_fields() {
         fs.jz = jkz.data(); fs.kx = kxd.data(); fs.pc = pcp.data(); fs.pd = pid.data(); fs.hc = hcg.data();
         fs.wl = wlo.data(); fs.wu = whi.data(); fs.g2 = gm2_b; fs.opb = opb; fs.ns = ns; fs.N = N; fs.a = a;
     }
-    if (sp) {
-        if (yf)
-            sponge_pack(g, Rx.data(), Ry.data(), jkz.data(), hcg.data(), wlo.data(), whi.data(), gm2_b, opb, S1.data(),
-                        S2.data());
-        else fh_sponge_psi(fs, L, Rx.data(), Ry.data(), S1.data(), S2.data());
-        fft_run(fft, S1.data(), ns, true);
-        sponge_mask(g, S1.data(), maskx.data(), masky_n.data(), masky_h.data(), ns);
-        fft_run(fft, S1.data(), ns, false);
-        if (!yf) fh_sponge_unpack(fs, L, S1.data(), S2.data(), Rx.data(), Ry.data());
-    }
-    // the FP32-mixed form: the three planes of the real fields transformed in FP32 (F is float in both forms)
-    bool ions = false;
-    for (const auto& is : cfg.ions) ions = ions || cfg.loaded(is);
-    const bool f32 = cfg.mixed && yf && !ions && g.cm;
-    cxf* T3f = f32 ? reinterpret_cast<cxf*>(T3.data()) : nullptr;
-    fields_pack3(g, sp && yf ? S1.data() : nullptr, S2.data(), opb, Rx.data(), Ry.data(), Lx.data(), Ly.data(),
-                 Ez.data(), Bz.data(), T3.data(), ts, ns, T3f);
-    if (f32) {
-        fft_run_f(fft, T3f, 3 * ns, true);
-        fields_to_F_f(T3f, ts, F.data(), long(ns + 2) * nk, nk, ns);
+    const long fpl = long(ns + 2) * nk;
+    if (yf) {
+        if (sp)
+            sponge_R(g, fft, Rx.data(), Ry.data(), jkz.data(), hcg.data(), wlo.data(), whi.data(), gm2_b, opb, maskx.data(),
+                     masky_n.data(), masky_h.data(), S1.data(), S2.data());
+        // the FP32-mixed form: the three planes of the real fields transformed in FP32 (F is float in both forms)
+        bool ions = false;
+        for (const auto& is : cfg.ions) ions = ions || cfg.loaded(is);
+        if (cfg.mixed && !ions && g.cm)
+            real_fields_f(g, fft, Rx.data(), Ry.data(), Lx.data(), Ly.data(), Ez.data(), Bz.data(),
+                          reinterpret_cast<cxf*>(T3.data()), ts, F.data(), fpl, ns);
+        else
+            real_fields(g, fft, Rx.data(), Ry.data(), Lx.data(), Ly.data(), Ez.data(), Bz.data(), T3.data(), ts, F.data(),
+                        fpl, ns);
     } else {
+        if (sp) {
+            fh_sponge_psi(fs, L, Rx.data(), Ry.data(), S1.data(), S2.data());
+            fft_run(fft, S1.data(), ns, true);
+            sponge_mask(g, S1.data(), maskx.data(), masky_n.data(), masky_h.data(), ns);
+            fft_run(fft, S1.data(), ns, false);
+            fh_sponge_unpack(fs, L, S1.data(), S2.data(), Rx.data(), Ry.data());
+        }
+        fields_pack3(g, nullptr, S2.data(), opb, Rx.data(), Ry.data(), Lx.data(), Ly.data(), Ez.data(), Bz.data(),
+                     T3.data(), ts, ns);
         fft_run(fft, T3.data(), 3 * ns, true);
-        fields_to_F(T3.data(), ts, F.data(), long(ns + 2) * nk, nk, ns);
+        fields_to_F(T3.data(), ts, F.data(), fpl, nk, ns);
     }
     toc(F_SPONGE);
 }
@@ -1133,6 +1136,11 @@ void Sim::real_fields_slice(int n) {
     ensure_layout(false, false);
     const SpecGeom g = geom();
     const long l = n - a;
+    if (yf) {
+        real_fields(g, fft, Rx.data() + l * nk, Ry.data() + l * nk, Lx.data() + l * nk, Ly.data() + l * nk,
+                    Ez.data() + l * nk, Bz.data() + l * nk, tp3.data(), nk, F.data() + l * nk, long(ns + 2) * nk, 1);
+        return;
+    }
     fields_pack3(g, nullptr, nullptr, 0, Rx.data() + l * nk, Ry.data() + l * nk, Lx.data() + l * nk, Ly.data() + l * nk,
                  Ez.data() + l * nk, Bz.data() + l * nk, tp3.data(), nk, 1);
     fft_run(fft, tp3.data(), 3, true);

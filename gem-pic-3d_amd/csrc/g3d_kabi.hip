@@ -189,10 +189,7 @@ int g3d_real_fields_slice(const g3d_spec_ctx* c, const g3d_cpx* Rx, const g3d_cp
         g3d::need(Ez, "Ez"); g3d::need(Bz, "Bz"); g3d::need(F_slice, "F"); g3d::need(scratch, "scratch");
         const g3d::SpecGeom g = g3d::geom_of(*c);
         if (fpl < g.nk) throw std::invalid_argument("g3d_real_fields_slice: fpl below nk");
-        g3d::fields_pack3(g, nullptr, nullptr, 0, const_cast<g3d::cx*>(Rx), const_cast<g3d::cx*>(Ry), Lx, Ly, Ez, Bz,
-                          scratch, g.nk, 1);
-        g3d::fft_run(c->plan->p, scratch, 3, true);
-        g3d::fields_to_F(scratch, g.nk, F_slice, fpl, g.nk, 1);
+        g3d::real_fields(g, c->plan->p, Rx, Ry, Lx, Ly, Ez, Bz, scratch, g.nk, F_slice, fpl, 1);
     });
 }
 
@@ -231,15 +228,9 @@ int g3d_sponge_real_fields(const g3d_spec_ctx* c, int sponge, const double* mask
         g3d::cx* S2 = scratch + ts;
         g3d::cx* T3 = scratch + 2 * ts;
         const double opb = 1 + beta_b;
-        if (sponge) {
-            g3d::sponge_pack(g, Rx, Ry, jkz, c->hcg, c->wlo, c->whi, gm2_b, opb, S1, S2);
-            g3d::fft_run(c->plan->p, S1, g.ns, true);
-            g3d::sponge_mask(g, S1, maskx, masky, masky, g.ns);
-            g3d::fft_run(c->plan->p, S1, g.ns, false);
-        }
-        g3d::fields_pack3(g, sponge ? S1 : nullptr, S2, opb, Rx, Ry, Lx, Ly, Ez, Bz, T3, ts, g.ns);
-        g3d::fft_run(c->plan->p, T3, 3 * g.ns, true);
-        g3d::fields_to_F(T3, ts, F, long(g.ns + 2) * g.nk, g.nk, g.ns);
+        if (sponge)
+            g3d::sponge_R(g, c->plan->p, Rx, Ry, jkz, c->hcg, c->wlo, c->whi, gm2_b, opb, maskx, masky, masky, S1, S2);
+        g3d::real_fields(g, c->plan->p, Rx, Ry, Lx, Ly, Ez, Bz, T3, ts, F, long(g.ns + 2) * g.nk, g.ns);
     });
 }
 
