@@ -770,13 +770,17 @@ void Sim::currents() {
     d.dy = dy; d.nh = ns + 3; d.a = a; d.N = N; d.nx = cfg.nx; d.ny = cfg.ny; d.yf = yf; d.nk = nk;
     bunch_deposit(d, beam.view(), np, dep_scratch);
     const SpecGeom g = geom();
-    currents_zfilter(g, jw.data(), hcg.data(), cfg.zeta_filter, zax.uniform, S1.data(), jkz.data());
-    fft_run(fft, S1.data(), ns + 1, false);
-    fft_run(fft, jkz.data(), ns + 1, false);
     const bool keep0 = cfg.plasma_on && cfg.box_mean && !starting_;
-    if (yf) currents_unpack(g, S1.data(), jkx.data(), jky.data(), jkz.data(), keep0);
-    else fh_currents(S1.data(), jkx.data(), jky.data(), jkz.data(), ns + 1, lview(0.0), filt.data(), cfg.k_filter,
-                     keep0, cfg.Ly);
+    if (yf)
+        current_spectra(g, fft, jw.data(), hcg.data(), cfg.zeta_filter, zax.uniform, S1.data(), jkx.data(), jky.data(),
+                        jkz.data(), keep0);
+    else {
+        currents_zfilter(g, jw.data(), hcg.data(), cfg.zeta_filter, zax.uniform, S1.data(), jkz.data());
+        fft_run(fft, S1.data(), ns + 1, false);
+        fft_run(fft, jkz.data(), ns + 1, false);
+        fh_currents(S1.data(), jkx.data(), jky.data(), jkz.data(), ns + 1, lview(0.0), filt.data(), cfg.k_filter, keep0,
+                    cfg.Ly);
+    }
     toc(F_CUR);
 }
 

@@ -95,15 +95,17 @@ bool tile_index_fit(TileIndex& t, long n, long ntile) {
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     return ok;
 }
-// Whether a half-cell is streamed through tiles: from kTiledMin particles on (below, the binning launches cost more than
-// the windows save: with the spectra of the current, 1.6 x 10^4 particles at 1 per cell take 30 us untiled and 36 tiled,
-// 2.5 x 10^4 at 6 per cell 47 and 43, 2.6 x 10^5 at 4 per cell 290 and 66, where the untiled atomics meet in few
-// nodes), on a periodic grid that holds the tiles, with both field slices present.  The results are the
-// untiled kernel's but for the order of the current's sums, which its atomics leave free as well
-constexpr long kTiledMin = 20000;
+// Whether a half-cell is streamed through tiles, where binning the list (three launches) costs less than the windows
+// save: from kTiledMin particles on when they are at least 3 for 2 points (untiled, the atomics of the particles of a cell
+// meet in its nodes), else from kTiledSparse on.  With the spectra of the current, untiled and tiled: 1.6 x 10^4
+// particles at 2 per cell 34 and 36 us, 2.5 x 10^4 at 3 per cell 46 and 40, 3.3 x 10^4 at 1 per cell 35 and 38,
+// 6.6 x 10^4 at 1 per cell 63 and 49, 2.6 x 10^5 at 4 per cell 290 and 66.  Periodic grids that hold the tiles, with both
+// field slices present.  The results are the untiled kernel's but for the order of the current's sums, which its
+// atomics leave free as well
+constexpr long kTiledMin = 20000, kTiledSparse = 49152;
 bool tiled_halfcell(const StreamArgs& a, long n, TileGeom& tg) {
     const FieldView& F = a.fv;
-    if (n < kTiledMin || n > kTileIndexMax || F.yf != 1 || a.n < F.a || a.n - F.a > F.ns) return false;
+    if (n < kTiledMin || (n < kTiledSparse && 2 * n < 3 * F.nk) || n > kTileIndexMax || F.yf != 1 || a.n < F.a || a.n - F.a > F.ns) return false;
     if (!(F.dx > 0) || !(F.dy > 0) || !tile_shape(tg, F.nx, F.ny, true, 3) || tg.ntile > 4096) return false;
     tg.fwin = 1; tg.block = 512; tg.aflush = 1;
     return true;
@@ -208,10 +210,7 @@ int g3d_bunch_currents(const g3d_spec_ctx* c, const g3d_axis* zax, const double*
         d.hcg = c->hcg; d.ia = ia; d.id = id ? id : ia; d.J = jw; d.dx = dx; d.dy = dy;
         d.nh = g.ns + 3; d.a = g.a; d.N = g.N; d.nx = g.nx; d.ny = g.ny; d.yf = 1; d.nk = g.nk;
         if (np > 0) g3d::bunch_deposit(d, *p, np, g3d::deposit_scratch());
-        g3d::currents_zfilter(g, jw, c->hcg, zfilter, zuniform, scratch, jkz);
-        g3d::fft_run(c->plan->p, scratch, g.ns + 1, false);
-        g3d::fft_run(c->plan->p, jkz, g.ns + 1, false);
-        g3d::currents_unpack(g, scratch, jkx, jky, jkz, c->keep0);
+        g3d::current_spectra(g, c->plan->p, jw, c->hcg, zfilter, zuniform, scratch, jkx, jky, jkz, c->keep0);
     });
 }
 

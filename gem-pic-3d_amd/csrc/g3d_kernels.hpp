@@ -111,8 +111,9 @@ struct DepositArgs {
 // scratch of the ordered deposit (records, their sorted copies, the sort's temporary storage)
 struct DepositScratch {
     DevBuf<unsigned long long> key0, key1;
+    DevBuf<unsigned> k0, k1;         // the keys of the particle sort
     DevBuf<unsigned> rec0, rec1;
-    DevBuf<double> val, vs;          // the record values, and the same in sorted order
+    DevBuf<double> val, vs;          // the record values, and the same in sorted order (particle sort: the particles)
     DevBuf<unsigned char> tmp;
     DevBuf<long> runs;               // the long runs of equal keys: (first record, end) pairs
     DevBuf<int> nruns;
@@ -201,6 +202,9 @@ struct SpecGeom {
     const double *kx, *ky, *kxs, *kys, *filt, *filty;
     int cm = 0;      // sponge and real fields: R, L, E_z, B_z and jk column-major (mode ix ny + j); scratch row-major
 };
+// Fourier y, the two functions below fused with the transforms (g3d_sponge.hip): jw -> jk (S1: ns+1 planes of scratch)
+void current_spectra(const SpecGeom& g, const FftPlan& p, const double* jw, const double* hcg, int zfilter, int zuniform,
+                     cx* S1, cx* jkx, cx* jky, cx* jkz, int keep0);
 // currents: zeta filter of jw into S1 (jx + i jy) and jkz (jz + 0 i), ns+1 half-cell planes
 void currents_zfilter(const SpecGeom& g, const double* jw, const double* hcg, int zfilter, int zuniform, cx* S1, cx* jkz);
 // unpack the pair, transverse filter, k = 0 rule

@@ -245,6 +245,94 @@ __global__ void __launch_bounds__(kT) k_rows_F(const C* T, long ts, float* F, lo
     }
 }
 
+// ---------------------------------------------------------------- currents (src/sim_particles.cpp:120-158)
+//   k_cur_rows   the (1,2,1)/4 zeta filter of the deposit, j_x + i j_y and j_z of a row, x transforms
+//   k_cur_cols   y transforms of a tile of columns (S1: in pairs kx, nx - kx), the packed pair unpacked, the filter
+// 129 half-cells of 256 x 256: 445 us as filter, two 2D transforms and unpack, now 340 (two transforms move 270 MB each way)
+struct CurView {
+    int nx, ny, lx, ly, ns, N, a, zf, zu, keep0;
+    long nk;
+    const double *J, *hc, *filt, *filty;
+    const cx *twx, *twy;
+    cx *s1, *jx, *jy, *jz;
+};
+__global__ void __launch_bounds__(kT) k_cur_rows(CurView g, int rpw) {
+    extern __shared__ __align__(16) unsigned char smraw[];
+    cx* buf = reinterpret_cast<cx*>(smraw);
+    const int nx = g.nx, sp = padded(nx);
+    cx* tws = buf + size_t(2 * rpw) * sp;
+    load_twiddles(tws, g.twx, nx >> 1, false);
+    const long row0 = long(blockIdx.x) * rpw, left = (long(g.ns + 1) << g.ly) - row0;
+    const int nr = left < rpw ? int(left) : rpw, tot = nr << g.lx, nh = g.ns + 3;
+    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
+        const int r = e >> g.lx, i = e & (nx - 1);
+        const long row = row0 + r;
+        const int hk = int(row >> g.ly), hc_ = g.a - 1 + hk, hw = hk + 1;
+        const long ip = ((row & (g.ny - 1)) << g.lx) + i;
+        double v[3] = {0, 0, 0};
+        if (hc_ >= 0 && hc_ <= g.N - 2)
+#pragma unroll
+            for (int comp = 0; comp < 3; ++comp) {
+                const double* Jc = g.J + size_t(comp) * nh * g.nk;
+                const double mid = Jc[hw * g.nk + ip];
+                if (!g.zf) { v[comp] = mid; continue; }
+                const double lo = Jc[(hw - 1) * g.nk + ip], hi = Jc[(hw + 1) * g.nk + ip];
+                v[comp] = g.zu ? 0.25 * lo + 0.5 * mid + 0.25 * hi
+                               : (0.25 * g.hc[hc_ + 1] * lo + 0.5 * g.hc[hc_ + 2] * mid + 0.25 * g.hc[hc_ + 3] * hi) / g.hc[hc_ + 2];
+            }
+        const int b = lpos(bitrev(i, g.lx));
+        buf[2 * r * sp + b] = mk(v[0], v[1]);
+        buf[(2 * r + 1) * sp + b] = mk(v[2], 0);
+    }
+    __syncthreads();
+    lds_fft(buf, nx, g.lx, 2 * nr, sp, tws);
+    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
+        const int r = e >> g.lx, i = e & (nx - 1);
+        const long o = (row0 << g.lx) + e;
+        g.s1[o] = buf[2 * r * sp + lpos(i)];
+        g.jz[o] = buf[(2 * r + 1) * sp + lpos(i)];
+    }
+}
+// The first npair workgroups: 2^lpw column pairs of S1 (pair m: columns m and nx - m, each the other's mirror; m = 0:
+// columns 0 and nx/2, each its own); the others: 2 * 2^lpw adjacent columns of j_z
+__global__ void __launch_bounds__(kT) k_cur_cols(CurView g, int lpw, long npair) {
+    extern __shared__ __align__(16) unsigned char smraw[];
+    cx* buf = reinterpret_cast<cx*>(smraw);
+    const int ny = g.ny, sp = padded(ny), pw = 1 << lpw;
+    cx* tws = buf + size_t(2 * pw) * sp;
+    load_twiddles(tws, g.twy, ny >> 1, false);
+    const int per = (g.nx / 2) >> lpw;
+    const bool pairs = blockIdx.x < npair;
+    // the tiles of one XCD consecutive (workgroup b runs on XCD b mod 8): the 64-byte runs of neighbours meet in its L2
+    const long w = row_block(int(pairs ? blockIdx.x : blockIdx.x - npair), int(npair), 1), p = w / per;
+    const int m0 = int(w - p * per) << lpw, tot = 2 * pw * ny;
+    const long pl = p * g.nk;
+    auto col = [&](int q) {
+        if (!pairs) return 2 * m0 + q;
+        const int m = m0 + (q & (pw - 1));
+        return q < pw ? m : (m ? g.nx - m : g.nx / 2);
+    };
+    auto factor = [&](int x, int j) { return (x == 0 && j == 0 && !g.keep0) ? 0.0 : g.filt[x] * g.filty[j]; };
+    const cx* A = pairs ? g.s1 : g.jz;
+    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
+        const int j = e >> (lpw + 1), q = e & (2 * pw - 1);
+        buf[q * sp + lpos(bitrev(j, g.ly))] = A[pl + (long(j) << g.lx) + col(q)];
+    }
+    __syncthreads();
+    lds_fft(buf, ny, g.ly, 2 * pw, sp, tws);
+    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
+        const int j = e >> (lpw + 1), q = e & (2 * pw - 1), x = col(q);
+        const double f = factor(x, j);
+        const long o = pl + (long(j) << g.lx) + x;
+        const cx z = buf[q * sp + lpos(j)];
+        if (!pairs) { g.jz[o] = f * z; continue; }
+        const int qm = m0 + (q & (pw - 1)) ? q ^ pw : q;
+        cx X, Y;
+        unpack_pair(z, conjg(buf[qm * sp + lpos((ny - j) & (ny - 1))]), X, Y);
+        g.jx[o] = f * X; g.jy[o] = f * Y;
+    }
+}
+
 int ilog(long n) { int l = 0; while ((1L << l) < n) ++l; return l; }
 // sequences of length n per workgroup: about kTile values, fewer where the grid would fall below 512 workgroups, at
 // least `least` (contiguous runs of a column tile)
@@ -310,6 +398,22 @@ void real_fields(const SpecGeom& g, const FftPlan& p, const cx* Rx, const cx* Ry
 void real_fields_f(const SpecGeom& g, const FftPlan& p, const cx* Rx, const cx* Ry, const cx* Lx, const cx* Ly,
                    const cx* Ez, const cx* Bz, cxf* T, long ts, float* F, long fpl, int count) {
     real_fields_t<cxf, float>(g, p, Rx, Ry, Lx, Ly, Ez, Bz, T, ts, F, fpl, count);
+}
+
+void current_spectra(const SpecGeom& g, const FftPlan& p, const double* jw, const double* hcg, int zf, int zu, cx* S1,
+                     cx* jkx, cx* jky, cx* jkz, int keep0) {
+    CurView c{g.nx, g.ny, ilog(g.nx), ilog(g.ny), g.ns, g.N, g.a, zf, zu, keep0, g.nk, jw, hcg, g.filt, g.filty, p.twx, p.twy,
+              S1, jkx, jky, jkz};
+    const long rows = long(g.ns + 1) * g.ny;
+    const int rpw = std::max(1, sequences(g.nx, 2 * rows, 1) / 2);
+    hipLaunchKernelGGL(k_cur_rows, dim3(blocks_for(rows, rpw)), dim3(lanes(2L * rpw * g.nx)),
+                       (size_t(2 * rpw) * (g.nx + g.nx / 8) + g.nx / 2) * sizeof(cx), stream(), c, rpw);
+    int pw = 1;
+    while (2 * pw < g.nx / 2 + 1 && 4 * pw * g.ny <= kTile && pw < 8) pw <<= 1;
+    const long npair = long(g.ns + 1) * ((g.nx / 2) / pw);
+    hipLaunchKernelGGL(k_cur_cols, dim3(unsigned(2 * npair)), dim3(lanes(2L * pw * g.ny)),
+                       (size_t(2 * pw) * (g.ny + g.ny / 8) + g.ny / 2) * sizeof(cx), stream(), c, ilog(pw), npair);
+    launch_check("current spectra");
 }
 
 }  // namespace g3d
