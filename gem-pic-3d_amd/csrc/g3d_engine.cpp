@@ -1248,9 +1248,11 @@ void Sim::march_plasma(double s0, double s1) {
     // FP32-mixed: the tile workgroups XCD-contiguous (G3D_STREAM_XCD=0: in tile order; the FP64 kernel ran 4 %
     // slower so)
     { const char* ex = getenv("G3D_STREAM_XCD"); tg.xcd = mx && (ex ? atoi(ex) : 1) && tg.ntile % 8 == 0 && tg.ntile < (1L << 30); }
-    // FP32-mixed: the tile windows go to the current planes with float atomics instead of slabs (3 % faster at
-    // 256 x 256: the row kernel then reads one plane set); G3D_STREAM_AFLUSH=0 keeps the slabs
-    { const char* e = getenv("G3D_STREAM_AFLUSH"); tg.aflush = (mx && !(e && atoi(e) == 0)) || mxi; }
+    // the tile windows go to the current planes with atomics instead of slabs: the row kernel then reads one plane set.
+    // FP32-mixed: 3 % of a step at 256 x 256; FP64, 4 a cell: rows 8.1 -> 4.5 us against 14.2 -> 14.7 of the stream at
+    // 64 x 64, 8.6 -> 4.9 against 15.4 -> 16.0 at 128 x 128, 10.1 -> 6.5 against 27.5 -> 28.7 at 256 x 256.
+    // G3D_STREAM_AFLUSH=0 keeps the slabs
+    { const char* e = getenv("G3D_STREAM_AFLUSH"); tg.aflush = !(e && atoi(e) == 0) || mxi; }
     // FP32-mixed: tiles denser than G3D_STREAM_CHUNK (default 1) times one workgroup's lanes are streamed in
     // chunks of that many particles (0: off)
     const char* ech = getenv("G3D_STREAM_CHUNK");
@@ -1402,7 +1404,7 @@ void Sim::march_plasma(double s0, double s1) {
             }
             tic(F_SFFT);
             TileGeom tr = tg;
-            if (tg.fh) tr.ntile = 0;             // free-hand: the windows are already in jsr
+            if (tg.fh || tg.aflush) tr.ntile = 0;      // the windows are already in jsr
             pass_rows_fwd(jsr.data(), tr, fft, sp3.data(), last ? rho_lines.data() + long(n) * (nx + ny) : nullptr,
                           last && rho_lines_i.size() ? rho_lines_i.data() + long(n) * (nx + ny) : nullptr, i0, j0, cm);
             toc(F_SFFT);

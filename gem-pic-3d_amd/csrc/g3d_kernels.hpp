@@ -46,7 +46,7 @@ struct StreamArgs {
 
 // Transverse tiles of the streaming list: the fresh plasma is loaded tile by tile (TX x TY cells), particles
 // [off[t], off[t+1]) belong to tile t.  A tile's workgroup deposits into an LDS window of WX x WY nodes starting
-// at node (tx TX - 1 - M, ty TY - 1 - M) and writes it to its slab (5 planes of WX x WY); deposits that leave the
+// at node (tx TX - 1 - M, ty TY - 1 - M) and adds it to jsr (aflush), or writes it to its slab (5 planes of WX x WY); deposits that leave the
 // window go to jsr with global atomics.  Particles from off[ntile] on (joining, freed) are not tiled.
 struct TileGeom {
     int TX, TY, M, WX, WY, ntx, nty;
@@ -57,7 +57,7 @@ struct TileGeom {
     // further chunks of a tile, xtile/xstart[0 .. *xcount), run in max_extra more workgroups after the tiles and
     // add their window to the current planes with atomics
     int chunk, max_extra;
-    int aflush;                       // FP32-mixed: every window added to the current planes with atomics (no slabs)
+    int aflush;                       // every window added to the current planes with atomics (no slabs)
     // FP32-mixed: tile workgroups XCD-contiguous (workgroup b runs on XCD b mod 8; with max_extra and ntile
     // multiples of 8, XCD x takes tiles x ntile/8 ... (x+1) ntile/8 - 1, so the overlapping field windows of
     // neighbouring tiles meet in one L2)
