@@ -38,6 +38,53 @@ __device__ __forceinline__ void tsc_wd(double x, double d, int n, int idx[3], do
     dw[2] = (0.5 + f) / d;
 }
 
+// ---------------------------------------------------------------- sums of a workgroup's neighbouring particles in LDS
+// Lists keep neighbours in space together, so the stencils of a workgroup's kBoxT consecutive particles cover a small box
+// of nodes: their contributions are added in LDS and the box goes to the planes once, one atomic per node and plane.  With
+// a global atomic per contribution (108 per particle of the reverse, 36 of the push) these bound both kernels, at 34 x 10^9
+// atomics a second: 32768 particles on 128 x 128 nodes took 105 us and 36 us, now 67 us and 16 us, and 8192 on 64 x 64 in
+// the reverse 31 us, now 25 us (there the chain of a particle's operations bounds it).  128 lanes: 64 hold half the
+// particles a node, and 256 leave half of the CUs idle at these sizes.  A box beyond the LDS (a list in no order) takes
+// the global atomics.
+constexpr int kBoxT = 128;
+struct NodeBox {
+    int x0, y0, W, H;                // W = 0: no box
+};
+// the box of the stencils whose middle nodes are (ix, jn) (of the lanes with on), relative to the first particle's so
+// that it may cross the periodic edge; every lane of the workgroup calls it
+__device__ __forceinline__ NodeBox node_box(bool on, int ix, int jn, int nx, int ny, int cap) {
+    __shared__ int red[kBoxT / 64][4], ref[2];
+    if (threadIdx.x == 0) { ref[0] = ix; ref[1] = jn; }
+    __syncthreads();
+    auto near = [](int d, int n) { d = wrap_index(d, n); return d >= n - n / 2 ? d - n : d; };
+    int v[4] = {1 << 30, 1 << 30, 1 << 30, 1 << 30};        // minima of u, v, -u, -v
+    if (on) { v[0] = near(ix - ref[0], nx); v[1] = near(jn - ref[1], ny); v[2] = -v[0]; v[3] = -v[1]; }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { const int t = __shfl_xor(v[k], o, 64); v[k] = t < v[k] ? t : v[k]; }
+    if ((threadIdx.x & 63) == 0)
+        for (int k = 0; k < 4; ++k) red[threadIdx.x >> 6][k] = v[k];
+    __syncthreads();
+    for (int k = 0; k < 4; ++k)
+        for (int w = 0; w < kBoxT / 64; ++w) v[k] = red[w][k] < v[k] ? red[w][k] : v[k];
+    if (v[0] == 1 << 30) return NodeBox{0, 0, 0, 0};         // nothing to add
+    const int W = -v[2] - v[0] + 3, H = -v[3] - v[1] + 3;
+    if (long(W) * H > cap) return NodeBox{0, 0, 0, 0};
+    return NodeBox{ref[0] + v[0] - 1, ref[1] + v[1] - 1, W, H};
+}
+// the middle node of a wrapped coordinate's stencil
+__device__ __forceinline__ int mid_node(double x, double d, int n) { return wrap_index(int(floor(x / d + 0.5)), n); }
+// plane p of the box in LDS to the global plane
+__device__ __forceinline__ void box_flush(const NodeBox& b, const double* acc, double* plane, int nx, int ny) {
+    for (int r = threadIdx.x; r < b.W * b.H; r += blockDim.x) {
+        const double v = acc[r];
+        if (v == 0) continue;
+        const int j = r / b.W, u = r - j * b.W;
+        atomicAdd(&plane[long(wrap_index(b.y0 + j, ny)) * nx + wrap_index(b.x0 + u, nx)], v);
+    }
+}
+
 // ---------------------------------------------------------------- the push on T = double or Dn
 template <typename T>
 struct SP { T x, y, zeta, z, px, py, pz; };
@@ -151,19 +198,16 @@ __device__ __forceinline__ double gather_comp(const g3d_spush_ctx& c, const Gath
     return s;
 }
 
-__global__ void __launch_bounds__(kT) k_spush(g3d_spush_ctx c) {
+constexpr int kPushNodes = 1024;             // nodes of a push's box: 5 planes, 40 KB
+__global__ void __launch_bounds__(kBoxT) k_spush(g3d_spush_ctx c) {
+    __shared__ double acc[5 * kPushNodes];
     const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= c.np) return;
     const long nk = long(c.nx) * c.ny;
-    SP<double> p{c.x[i], c.y[i], c.zeta[i], c.z[i], c.px[i], c.py[i], c.pz[i]};
-    int alive = c.alive[i];
-    auto gather = [&](double xg, double yg, double zm, double E[3], double B[3]) {
-        const GatherPoint g = gather_point(c, xg, yg, zm);
-        double v[6];
-        for (int comp = 0; comp < 6; ++comp) v[comp] = gather_comp(c, g, comp, nullptr, nullptr, nullptr);
-        E[0] = v[0]; E[1] = v[1]; E[2] = v[2]; B[0] = v[3]; B[1] = v[4]; B[2] = v[5];
-    };
+    // the first deposit of a particle waits for the box; the second (a trapped electron's beam current) is rare
+    struct Dep { double x, y, f, vx, vy, vz; } d{};
+    int nd = 0;
     auto deposit = [&](double x, double y, double f, double vx, double vy, double vz) {
+        if (nd++ == 0) { d = Dep{x, y, f, vx, vy, vz}; return; }
         int ix[3], jn[3]; double wx[3], wn[3];
         tsc_periodic(x, c.dx, c.nx, ix, wx);
         tsc_periodic(y, c.dy, c.ny, jn, wn);
@@ -178,9 +222,46 @@ __global__ void __launch_bounds__(kT) k_spush(g3d_spush_ctx c) {
                 atomicAdd(&c.J[cq * nk + k], ww);
             }
     };
-    tpush<double>(c, p, c.q[i], c.qm[i], c.w[i], alive, gather, deposit);
-    c.x[i] = p.x; c.y[i] = p.y; c.zeta[i] = p.zeta; c.z[i] = p.z; c.px[i] = p.px; c.py[i] = p.py; c.pz[i] = p.pz;
-    c.alive[i] = alive;
+    if (i < c.np) {
+        SP<double> p{c.x[i], c.y[i], c.zeta[i], c.z[i], c.px[i], c.py[i], c.pz[i]};
+        int alive = c.alive[i];
+        auto gather = [&](double xg, double yg, double zm, double E[3], double B[3]) {
+            const GatherPoint g = gather_point(c, xg, yg, zm);
+            double v[6];
+            for (int comp = 0; comp < 6; ++comp) v[comp] = gather_comp(c, g, comp, nullptr, nullptr, nullptr);
+            E[0] = v[0]; E[1] = v[1]; E[2] = v[2]; B[0] = v[3]; B[1] = v[4]; B[2] = v[5];
+        };
+        tpush<double>(c, p, c.q[i], c.qm[i], c.w[i], alive, gather, deposit);
+        c.x[i] = p.x; c.y[i] = p.y; c.zeta[i] = p.zeta; c.z[i] = p.z; c.px[i] = p.px; c.py[i] = p.py; c.pz[i] = p.pz;
+        c.alive[i] = alive;
+    }
+    const bool on = nd > 0;
+    const NodeBox b = node_box(on, mid_node(d.x, c.dx, c.nx), mid_node(d.y, c.dy, c.ny), c.nx, c.ny, kPushNodes);
+    const int n = b.W * b.H;
+    if (!b.W) { nd = 1; if (on) deposit(d.x, d.y, d.f, d.vx, d.vy, d.vz); return; }
+    for (int r = threadIdx.x; r < 5 * n; r += blockDim.x) acc[r] = 0;
+    __syncthreads();
+    if (on) {
+        int ix[3], jn[3]; double wx[3], wn[3];
+        tsc_periodic(d.x, c.dx, c.nx, ix, wx);
+        tsc_periodic(d.y, c.dy, c.ny, jn, wn);
+        const int u0 = wrap_index(ix[0] - b.x0, c.nx), v0 = wrap_index(jn[0] - b.y0, c.ny), cq = d.f < 0 ? 3 : 4;
+        if (u0 + 3 > b.W || v0 + 3 > b.H) { nd = 1; deposit(d.x, d.y, d.f, d.vx, d.vy, d.vz); }
+        else
+#pragma unroll
+        for (int v = 0; v < 3; ++v)
+#pragma unroll
+            for (int u = 0; u < 3; ++u) {
+                double* A = acc + (v0 + v) * b.W + u0 + u;
+                const double ww = d.f * wx[u] * wn[v] * c.ia;
+                atomicAdd(A, ww * d.vx);
+                atomicAdd(A + n, ww * d.vy);
+                atomicAdd(A + 2 * n, ww * d.vz);
+                atomicAdd(A + cq * n, ww);
+            }
+    }
+    __syncthreads();
+    for (int k = 0; k < 5; ++k) box_flush(b, acc + k * n, c.J + k * nk, c.nx, c.ny);
 }
 
 // The TSC weights of a point, their x and y derivatives and nodes (tsc_wd on both axes)
@@ -229,9 +310,9 @@ __device__ __forceinline__ void deposit_rev(const g3d_spush_ctx& c, const double
 // every statement transposed in reverse order; the Boris rotations through boris_rev.  The branch decisions and
 // the skipped deposit of a zero factor are the forward's.  Gives the same numbers as the forward-mode reverse on
 // 13-direction dual numbers, in registers (that one spilled 828 bytes per lane).
-__global__ void __launch_bounds__(kT) k_spush_vjp(g3d_spush_ctx c, g3d_spush_adj a) {
-    const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= c.np) return;
+// b: the box of the workgroup's gather stencils (acc: 12 planes, gF0 then gF1), or W = 0
+__device__ __forceinline__ void spush_vjp_one(const g3d_spush_ctx& c, const g3d_spush_adj& a, long i, const NodeBox& b,
+                                              double* acc) {
     const long nk = long(c.nx) * c.ny;
     const double x = c.x[i], y = c.y[i], zeta = c.zeta[i], z = c.z[i];
     const double p[3] = {c.px[i], c.py[i], c.pz[i]};
@@ -390,16 +471,29 @@ __global__ void __launch_bounds__(kT) k_spush_vjp(g3d_spush_ctx c, g3d_spush_adj
         // position derivatives on
         const GatherPoint gp = gather_point(c, twrap(xm, Lx), twrap(ym, Ly), zetam);
         double xmb = 0, ymb = 0, zetamb = 0;
+        const int nb = b.W * b.H;
+        const int u0 = wrap_index(int(gp.k[0] % c.nx) - b.x0, c.nx), v0 = wrap_index(int(gp.k[0] / c.nx) - b.y0, c.ny);
+        const int r0 = v0 * b.W + u0;
+        const bool in = u0 + 3 <= b.W && v0 + 3 <= b.H;       // inside the box (never, without one)
         for (int comp = 0; comp < 6; ++comp) {
             const double e = comp < 3 ? Eb[comp] : Bb[comp - 3];
             double gxc, gyc, gzc;
             gather_comp(c, gp, comp, &gxc, &gyc, &gzc);
             xmb += e * gxc; ymb += e * gyc; zetamb += e * gzc;
             if (e == 0) continue;
-            for (int t = 0; t < 9; ++t) {
-                atomicAdd(&a.gF0[comp * nk + gp.k[t]], e * gp.w[t] * gp.gz);
-                atomicAdd(&a.gF1[comp * nk + gp.k[t]], e * gp.w[t] * gp.fz);
-            }
+            if (in) {
+                double* A = acc + comp * nb + r0;
+#pragma unroll
+                for (int t = 0; t < 9; ++t) {
+                    const int r = (t / 3) * b.W + t % 3;
+                    atomicAdd(A + r, e * gp.w[t] * gp.gz);
+                    atomicAdd(A + 6 * nb + r, e * gp.w[t] * gp.fz);
+                }
+            } else
+                for (int t = 0; t < 9; ++t) {
+                    atomicAdd(&a.gF0[comp * nk + gp.k[t]], e * gp.w[t] * gp.gz);
+                    atomicAdd(&a.gF1[comp * nk + gp.k[t]], e * gp.w[t] * gp.fz);
+                }
         }
         // zetam = zeta - hl / 2; xm = x + dt0 px / (2 g0); ym likewise
         zetas += zetamb;
@@ -422,6 +516,35 @@ __global__ void __launch_bounds__(kT) k_spush_vjp(g3d_spush_ctx c, g3d_spush_adj
     for (int k = 0; k < 3; ++k) pbv[k] += g0b * p[k] / g0;
     if (hmode == 1) zetas += hlb;                      // hl = zeta - zn
     out(xs, ys, zetas, zs_, pbv);
+}
+constexpr int kVjpNodes = 640;               // nodes of a reverse's box: 12 planes, 60 KB
+__global__ void __launch_bounds__(kBoxT) k_spush_vjp(g3d_spush_ctx c, g3d_spush_adj a) {
+    __shared__ double acc[12 * kVjpNodes];
+    const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
+    const long nk = long(c.nx) * c.ny;
+    bool on = false;
+    int ix = 0, jn = 0;
+    if (i < c.np) {                           // the middle node of the gather, as the reverse forms it
+        const double zeta = c.zeta[i], h = c.zn1 - c.zn;
+        const int al = c.alive[i];
+        on = al == 1 || (al == 6 && zeta > c.zn);
+        const double px = c.px[i], py = c.py[i], pz = c.pz[i];
+        const double hl = zeta >= c.zn1 - 1e-9 * h ? h : (zeta - c.zn > 0 ? zeta - c.zn : 0.0);
+        const double g0 = sqrt(1 + px * px + py * py + pz * pz), A0 = 1 + px * px + py * py, D0 = g0 * (g0 + pz);
+        const double dt0 = hl / (A0 / D0);
+        ix = mid_node(twrap(c.x[i] + 0.5 * dt0 * px / g0, c.nx * c.dx), c.dx, c.nx);
+        jn = mid_node(twrap(c.y[i] + 0.5 * dt0 * py / g0, c.ny * c.dy), c.dy, c.ny);
+    }
+    const NodeBox b = node_box(on, ix, jn, c.nx, c.ny, kVjpNodes);
+    const int n = b.W * b.H;
+    for (int r = threadIdx.x; r < 12 * n; r += blockDim.x) acc[r] = 0;
+    __syncthreads();
+    if (i < c.np) spush_vjp_one(c, a, i, b, acc);
+    __syncthreads();
+    for (int k = 0; k < 6; ++k) {
+        box_flush(b, acc + k * n, a.gF0 + k * nk, c.nx, c.ny);
+        box_flush(b, acc + (6 + k) * n, a.gF1 + k * nk, c.nx, c.ny);
+    }
 }
 
 // The tangent-linear push: the primal state and fields as k_spush (the state arrays are read, not written), the
@@ -484,7 +607,7 @@ int g3d_stream_push(const g3d_spush_ctx* c) {
     return g3d::guard([&] {
         if (!c || c->nx < 1 || c->ny < 1 || c->np < 0) throw std::invalid_argument("stream push: bad context");
         if (c->np == 0) return;
-        hipLaunchKernelGGL(k_spush, dim3(blocks_for(c->np, kT)), dim3(kT), 0, stream(), *c);
+        hipLaunchKernelGGL(k_spush, dim3(blocks_for(c->np, kBoxT)), dim3(kBoxT), 0, stream(), *c);
         launch_check("stream push");
     });
 }
@@ -493,7 +616,7 @@ int g3d_stream_push_vjp(const g3d_spush_ctx* c, const g3d_spush_adj* g) {
         if (!c || !g || c->nx < 1 || c->ny < 1 || c->np < 0)
             throw std::invalid_argument("stream push vjp: bad context");
         if (c->np == 0) return;
-        hipLaunchKernelGGL(k_spush_vjp, dim3(blocks_for(c->np, kT)), dim3(kT), 0, stream(), *c, *g);
+        hipLaunchKernelGGL(k_spush_vjp, dim3(blocks_for(c->np, kBoxT)), dim3(kBoxT), 0, stream(), *c, *g);
         launch_check("stream push vjp");
     });
 }
