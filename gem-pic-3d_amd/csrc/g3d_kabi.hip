@@ -95,17 +95,17 @@ bool tile_index_fit(TileIndex& t, long n, long ntile) {
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     return ok;
 }
-// Whether a half-cell is streamed through tiles, where binning the list (three launches) costs less than the windows
-// save: from kTiledMin particles on when they are at least 3 for 2 points (untiled, the atomics of the particles of a cell
-// meet in its nodes), else from kTiledSparse on.  With the spectra of the current, untiled and tiled: 1.6 x 10^4
-// particles at 2 per cell 34 and 36 us, 2.5 x 10^4 at 3 per cell 46 and 40, 3.3 x 10^4 at 1 per cell 35 and 38,
-// 6.6 x 10^4 at 1 per cell 63 and 49, 2.6 x 10^5 at 4 per cell 290 and 66.  Periodic grids that hold the tiles, with both
-// field slices present.  The results are the untiled kernel's but for the order of the current's sums, which its
-// atomics leave free as well
-constexpr long kTiledMin = 20000, kTiledSparse = 49152;
+// Whether a half-cell is streamed through tiles, which costs three launches for the index.  With the spectra of the
+// current, untiled (a workgroup's deposits summed in its box) and tiled, in us: lists in the order of their lattice
+// 6.6 x 10^4 particles at 4 per cell 30 and 44, 1.3 x 10^5 at 4 per cell 44 and 50, 2.0 x 10^5 at 3 per cell 53 and 61,
+// 2.6 x 10^5 at 4 per cell 65 and 67, 3.9 x 10^5 at 6 per cell 84 and 86; a list in no order keeps the tiled times but,
+// untiled, takes those of one atomic per deposit (290 for 2.6 x 10^5).  So from the length on where the order no longer
+// matters for the better.  Periodic grids that hold the tiles, with both field slices present.  The results are the
+// untiled kernel's but for the order of the current's sums, which its atomics leave free as well
+constexpr long kTiledMin = 200000;
 bool tiled_halfcell(const StreamArgs& a, long n, TileGeom& tg) {
     const FieldView& F = a.fv;
-    if (n < kTiledMin || (n < kTiledSparse && 2 * n < 3 * F.nk) || n > kTileIndexMax || F.yf != 1 || a.n < F.a || a.n - F.a > F.ns) return false;
+    if (n < kTiledMin || n > kTileIndexMax || F.yf != 1 || a.n < F.a || a.n - F.a > F.ns) return false;
     if (!(F.dx > 0) || !(F.dy > 0) || !tile_shape(tg, F.nx, F.ny, true, 3) || tg.ntile > 4096) return false;
     tg.fwin = 1; tg.block = 512; tg.aflush = 1;
     return true;

@@ -7,6 +7,7 @@
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "g3d_kernels.hpp"
+#include "g3d_nodebox.hpp"
 #include "g3d_runtime.hpp"
 
 namespace g3d {
@@ -632,8 +633,12 @@ constexpr int stream_waves(int YF, bool ION, bool LASER) { return YF == 1 && !IO
 
 // workgroups 0 .. ntile-1: the particles of one tile with the LDS window, written to the tile's slab at the end;
 // the following workgroups: the untiled particles from off[ntile] on, one per lane, global atomics
-// TILES: false for a list without tiles (the windows' code and registers left out: 35 us against 39 for 3.3 x 10^4
-// electrons)
+// TILES: false for a list without tiles (the windows' code and registers left out).  Fourier y: a workgroup's deposits
+// are summed in an LDS box around its particles' midpoints, where they fit one (a list in the order of its lattice); the
+// deposits that miss the box, or find none, take the global atomics, 36 per particle, which bounded the kernel.  With the
+// spectra of the current: 8.2 x 10^3 electrons at 2 per cell 31 -> 23 us, 3.3 x 10^4 at 2 per cell 49 -> 26, 2.0 x 10^5
+// at 3 per cell 216 -> 50; 4.1 x 10^3 at 1 per cell 25 -> 23 (a chain of loads and FP64 operations of one wave, 15 us)
+constexpr int kBoxNodes = 8;          // the largest box, per lane: 5 planes of 8 nodes, 20 KB for 64 lanes
 template <int YF, bool ION, bool LASER, bool TILES>
 __global__ void __launch_bounds__(kStreamBlockMax)
 __attribute__((amdgpu_waves_per_eu(TILES ? stream_waves(YF, ION, LASER) : 1))) k_stream_halfcell(StreamArgs c, Parts S, Parts D, long n,
@@ -689,6 +694,17 @@ __attribute__((amdgpu_waves_per_eu(TILES ? stream_waves(YF, ION, LASER) : 1))) k
         __syncthreads();
     }
     const double zn = c.zs[c.n];
+    NodeBox box{};
+    if (!TILES && YF == 1) {
+        const bool on = k < hi && (p.alive == 1 || (p.alive == 6 && p.zeta > zn));
+        const double h = c.zs[c.n + 1] - zn, g0 = sqrt(1 + p.px * p.px + p.py * p.py + p.pz * p.pz);
+        const double t = 0.5 * (p.zeta - zn < h ? p.zeta - zn : h) * (g0 + p.pz) / (1 + p.px * p.px + p.py * p.py);
+        box = node_box(on, mid_node(wrap_mod(p.x + t * p.px, F.Lx), F.dx, F.nx),
+                       mid_node(wrap_mod(p.y + t * p.py, F.Ly), F.dy, F.ny), F.nx, F.ny, int(hi - lo), kBoxNodes * blockDim.x);
+        for (int r = threadIdx.x; r < 5 * box.W * box.H; r += blockDim.x) dep[r] = 0;
+        w = Win{dep, nullptr, nullptr, box.x0, box.y0, box.W, box.H, fl, 0, 0};
+        __syncthreads();
+    }
     unsigned cnt = 0;
     while (k < hi) {
         cnt += pushed_through(p.alive, p.zeta, zn);
@@ -713,6 +729,20 @@ __attribute__((amdgpu_waves_per_eu(TILES ? stream_waves(YF, ION, LASER) : 1))) k
                 if (gy < 0 || gy >= F.ny) continue;
                 jadd(c, cc * F.nk + long(gy) * F.nx + wrap_index(x0 + u, F.nx), v);
             }
+    }
+    if (!TILES && YF == 1) {
+        __syncthreads();
+        const int nb = box.W * box.H;
+        const float iw = 1.0f / float(box.W);
+        for (int r = threadIdx.x; r < nb; r += blockDim.x) {
+            double s[5];
+#pragma unroll
+            for (int cc = 0; cc < 5; ++cc) s[cc] = dep[cc * nb + r];
+            const int q = box_node(box, iw, r, F.nx, F.ny);
+#pragma unroll
+            for (int cc = 0; cc < 5; ++cc)
+                if (s[cc] != 0) jadd(c, cc * F.nk + q, s[cc]);
+        }
     }
     if (c.npush) add_pushes(c.npush, cnt);
 }
@@ -927,9 +957,10 @@ void stream_halfcell(const StreamArgs& a, Parts src, Parts dst, long nstrm, cons
                      const LaunchTimer& lt) {
     if (nstrm <= 0) return;
     // tile workgroups of tg.block lanes, then the untiled tail in workgroups of the same size
-    // (a short untiled list in workgroups of one wave, whose few waves then spread over the compute units: a half-cell of
-    // 4 x 10^3 particles and its spectra 31.5 -> 26 us, from 8 x 10^3 on no faster)
-    const int bs = tg.ntile ? tg.block : (nstrm <= 6144 ? 64 : kT);
+    // (an untiled list in workgroups of one wave: Fourier y, 128 lanes are 1 to 4 us slower where the list has a part in
+    // no order, whose atomics the few waves of a larger workgroup hide less, and at most 2 us faster elsewhere; free-hand
+    // y, a short list's few waves then spread over the compute units)
+    const int bs = tg.ntile ? tg.block : (a.fv.yf || nstrm <= 6144 ? 64 : kT);
     if (bs < 64 || bs > kStreamBlockMax || bs % 64) throw std::runtime_error("stream half-cell: bad block size");
     const long tail_blocks = nstrm > tg.n_tiled ? long(blocks_for(nstrm - tg.n_tiled, bs)) : 0;
     // the deposit window (5 double planes, an even number of values), the field window (12 floats per node) and the
@@ -937,7 +968,7 @@ void stream_halfcell(const StreamArgs& a, Parts src, Parts dst, long nstrm, cons
     const size_t pl = size_t(tg.WX) * tg.WY;
     const size_t lds = tg.ntile ? ((5 * pl + 1) & ~size_t(1)) * sizeof(double) + (tg.fwin ? pl * 12 * sizeof(float) : 0) +
                                       (a.fv.yf ? 0 : size_t(tg.WY + 2) * sizeof(double))
-                                : 0;
+                                : (a.fv.yf ? size_t(5) * kBoxNodes * bs * sizeof(double) : 0);
     const dim3 grid(unsigned(tg.ntile + tail_blocks)), blk(bs);
     if (a.npush && long(grid.x) > a.npush_cap) throw std::runtime_error("stream half-cell: push counter too small");
     const bool ion = a.ions != nullptr;

@@ -15,6 +15,7 @@
 #include "g3d_boris_rev.hpp"
 #include "g3d_dual.hpp"
 #include "g3d_kernels.hpp"
+#include "g3d_nodebox.hpp"
 #include "g3d_runtime.hpp"
 
 namespace g3d {
@@ -39,49 +40,23 @@ __device__ __forceinline__ void tsc_wd(double x, double d, int n, int idx[3], do
 }
 
 // ---------------------------------------------------------------- sums of a workgroup's neighbouring particles in LDS
-// Lists keep neighbours in space together, so the stencils of a workgroup's kBoxT consecutive particles cover a small box
-// of nodes: their contributions are added in LDS and the box goes to the planes once, one atomic per node and plane.  With
-// a global atomic per contribution (108 per particle of the reverse, 36 of the push) these bound both kernels, at 34 x 10^9
-// atomics a second: 32768 particles on 128 x 128 nodes took 105 us and 36 us, now 67 us and 16 us, and 8192 on 64 x 64 in
-// the reverse 31 us, now 25 us (there the chain of a particle's operations bounds it).  128 lanes: 64 hold half the
-// particles a node, and 256 leave half of the CUs idle at these sizes.  A box beyond the LDS (a list in no order) takes
-// the global atomics.
+// (node_box): one global atomic per node and plane of the box of kBoxT consecutive particles.  With one per contribution
+// (108 per particle of the reverse, 36 of the push) these bound both kernels, at 34 x 10^9 atomics a second: 32768
+// particles on 128 x 128 nodes took 105 us and 36 us, now 67 us and 16 us, and 8192 on 64 x 64 in the reverse 31 us, now
+// 25 us (there the chain of a particle's operations bounds it).  128 lanes: 64 hold half the particles a node, and 256
+// leave half of the CUs idle at these sizes.  A box beyond the LDS (a list in no order) takes the global atomics.
 constexpr int kBoxT = 128;
-struct NodeBox {
-    int x0, y0, W, H;                // W = 0: no box
-};
-// the box of the stencils whose middle nodes are (ix, jn) (of the lanes with on), relative to the first particle's so
-// that it may cross the periodic edge; every lane of the workgroup calls it
-__device__ __forceinline__ NodeBox node_box(bool on, int ix, int jn, int nx, int ny, int cap) {
-    __shared__ int red[kBoxT / 64][4], ref[2];
-    if (threadIdx.x == 0) { ref[0] = ix; ref[1] = jn; }
-    __syncthreads();
-    auto near = [](int d, int n) { d = wrap_index(d, n); return d >= n - n / 2 ? d - n : d; };
-    int v[4] = {1 << 30, 1 << 30, 1 << 30, 1 << 30};        // minima of u, v, -u, -v
-    if (on) { v[0] = near(ix - ref[0], nx); v[1] = near(jn - ref[1], ny); v[2] = -v[0]; v[3] = -v[1]; }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) { const int t = __shfl_xor(v[k], o, 64); v[k] = t < v[k] ? t : v[k]; }
-    if ((threadIdx.x & 63) == 0)
-        for (int k = 0; k < 4; ++k) red[threadIdx.x >> 6][k] = v[k];
-    __syncthreads();
-    for (int k = 0; k < 4; ++k)
-        for (int w = 0; w < kBoxT / 64; ++w) v[k] = red[w][k] < v[k] ? red[w][k] : v[k];
-    if (v[0] == 1 << 30) return NodeBox{0, 0, 0, 0};         // nothing to add
-    const int W = -v[2] - v[0] + 3, H = -v[3] - v[1] + 3;
-    if (long(W) * H > cap) return NodeBox{0, 0, 0, 0};
-    return NodeBox{ref[0] + v[0] - 1, ref[1] + v[1] - 1, W, H};
+// the workgroup's particles
+__device__ __forceinline__ int box_lanes(const g3d_spush_ctx& c) {
+    const long rest = c.np - long(blockIdx.x) * kBoxT;
+    return rest < kBoxT ? int(rest) : kBoxT;
 }
-// the middle node of a wrapped coordinate's stencil
-__device__ __forceinline__ int mid_node(double x, double d, int n) { return wrap_index(int(floor(x / d + 0.5)), n); }
-// plane p of the box in LDS to the global plane
+// a plane of the box in LDS to the global plane
 __device__ __forceinline__ void box_flush(const NodeBox& b, const double* acc, double* plane, int nx, int ny) {
+    const float iw = 1.0f / float(b.W);
     for (int r = threadIdx.x; r < b.W * b.H; r += blockDim.x) {
         const double v = acc[r];
-        if (v == 0) continue;
-        const int j = r / b.W, u = r - j * b.W;
-        atomicAdd(&plane[long(wrap_index(b.y0 + j, ny)) * nx + wrap_index(b.x0 + u, nx)], v);
+        if (v != 0) atomicAdd(&plane[box_node(b, iw, r, nx, ny)], v);
     }
 }
 
@@ -236,7 +211,7 @@ __global__ void __launch_bounds__(kBoxT) k_spush(g3d_spush_ctx c) {
         c.alive[i] = alive;
     }
     const bool on = nd > 0;
-    const NodeBox b = node_box(on, mid_node(d.x, c.dx, c.nx), mid_node(d.y, c.dy, c.ny), c.nx, c.ny, kPushNodes);
+    const NodeBox b = node_box(on, mid_node(d.x, c.dx, c.nx), mid_node(d.y, c.dy, c.ny), c.nx, c.ny, box_lanes(c), kPushNodes);
     const int n = b.W * b.H;
     if (!b.W) { nd = 1; if (on) deposit(d.x, d.y, d.f, d.vx, d.vy, d.vz); return; }
     for (int r = threadIdx.x; r < 5 * n; r += blockDim.x) acc[r] = 0;
@@ -535,7 +510,7 @@ __global__ void __launch_bounds__(kBoxT) k_spush_vjp(g3d_spush_ctx c, g3d_spush_
         ix = mid_node(twrap(c.x[i] + 0.5 * dt0 * px / g0, c.nx * c.dx), c.dx, c.nx);
         jn = mid_node(twrap(c.y[i] + 0.5 * dt0 * py / g0, c.ny * c.dy), c.dy, c.ny);
     }
-    const NodeBox b = node_box(on, ix, jn, c.nx, c.ny, kVjpNodes);
+    const NodeBox b = node_box(on, ix, jn, c.nx, c.ny, box_lanes(c), kVjpNodes);
     const int n = b.W * b.H;
     for (int r = threadIdx.x; r < 12 * n; r += blockDim.x) acc[r] = 0;
     __syncthreads();

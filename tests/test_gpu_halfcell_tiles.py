@@ -1,5 +1,6 @@
-"""g3d_stream_halfcell on lists long enough to be streamed through tiles, against the same particles streamed in short
-lists (one atomic per deposit)."""
+"""g3d_stream_halfcell on lists long enough to be streamed through tiles, and on shorter ones in the order of a lattice
+(whose workgroups sum their deposits in a box), against the same particles streamed in short lists in no order (one
+atomic per deposit)."""
 import ctypes as C
 
 import numpy as np
@@ -27,9 +28,21 @@ def context(nx, ny, dx, dy, F, J, zs, ia, n, ns, s0, s1):
 
 
 # the tiles' shapes: 16 x 8 (512 x 64 cells are 256 of them), 8 x 8, a grid of two tiles across, one too small for tiles
-@pytest.mark.parametrize("nx,ny,count,in_place", [(512, 64, 70001, False), (64, 64, 20000, True), (32, 16, 20011, False),
-                                                  (8, 64, 20003, False), (128, 32, 25000, True)])
+@pytest.mark.parametrize("nx,ny,count,in_place", [(512, 64, 230001, False), (64, 64, 200000, True), (32, 16, 200011, False),
+                                                  (8, 64, 200003, False), (128, 32, 205000, True)])
 def test_tiled_halfcell_against_short_lists(nx, ny, count, in_place):
+    compare(nx, ny, count, in_place, False)
+
+
+# boxes across the periodic edge (rows of 2 per cell that begin in mid-row), as wide as the grid, a last workgroup of one
+# particle, less than a workgroup
+@pytest.mark.parametrize("nx,ny,count,in_place", [(128, 64, 16384, False), (32, 512, 30001, True), (16, 1024, 6401, False),
+                                                  (256, 32, 40, True)])
+def test_boxed_halfcell_against_no_order(nx, ny, count, in_place):
+    compare(nx, ny, count, in_place, True)
+
+
+def compare(nx, ny, count, in_place, ordered):
     r = np.random.default_rng(nx + ny)
     dx, dy, ns, n, h = 0.5, 0.7, 6, 2, 0.25
     zs = [h * k for k in range(ns)]
@@ -38,6 +51,10 @@ def test_tiled_halfcell_against_short_lists(nx, ny, count, in_place):
     # a few boxes away on either side, and on the edge itself
     p["x"] = nx * dx * r.uniform(-0.2, 1.2, count); p["y"] = ny * dy * r.uniform(-1.1, 1.1, count)
     p["x"][:3] = (0.0, nx * dx, -nx * dx)
+    if ordered:
+        k = np.arange(count) + nx
+        p["x"] = dx * (0.5 * k % nx + r.uniform(-0.6, 0.6, count))
+        p["y"] = dy * (0.5 * k // nx + r.uniform(-0.6, 0.6, count))
     p["px"], p["py"] = 0.5 * r.standard_normal((2, count))
     p["pz"] = np.abs(r.standard_normal(count))
     p["zeta"] = zs[n + 1]; p["z"] = 20 * r.uniform(size=count) ** 6
@@ -61,9 +78,11 @@ def test_tiled_halfcell_against_short_lists(nx, ny, count, in_place):
         return np.concatenate(out), J.get(np.float64).reshape(5, -1)
 
     got, Jg = stream([p])
-    want, Jw = stream([p[k:k + SHORT] for k in range(0, count, SHORT)])
-    assert (want["alive"] == 5).sum() > (p["alive"] == 5).sum() > 0
+    order = r.permutation(count) if ordered else np.arange(count)
+    want, Jw = stream([p[order][k:k + SHORT] for k in range(0, count, SHORT)])
+    want = want[np.argsort(order)]
+    assert count < 1000 or (want["alive"] == 5).sum() > (p["alive"] == 5).sum() > 0      # the input has trapped ones
     for f in ("x", "y", "zeta", "px", "py", "pz", "z", "q", "qm", "alive"):
         assert np.array_equal(got[f], want[f]), f
-    # sums of up to some hundred terms in another order
+    # sums of up to some thousand terms in another order
     assert np.abs(Jg - Jw).max() <= 1e-13 * np.abs(Jw).max()
