@@ -67,7 +67,7 @@ struct TileGeom {
     const int* xcount;
     // free-hand y: the tile rows follow the node table (cell j of a particle from fy; the last row of tiles may be
     // short), the windows stop at the walls, and the tile workgroups add their deposit window to the current
-    // planes with FP64 atomics instead of slabs (no field window)
+    // planes with atomics in any case
     int fh;
     Axis fy;
     long ntile, n_tiled;              // tiles; list entries binned (= off[ntile]); from n_tiled on: untiled tail
@@ -248,7 +248,7 @@ struct ModeArgs {
     double wex, qcorr, a2;
     int n, first, last, top, extrap, keep0, ny, kf;
 };
-// the fused kernels of a plasma pass (g3d_plasma.hip): rows forward (jsr + slabs -> X, 3 planes), columns
+// the fused kernels of a plasma pass (g3d_plasma.hip): rows forward (jsr, and slabs when tiles are given -> X, 3 planes), columns
 // (kind 0 pass, 1 front slice, 2 spectra only into jsn; X -> T, 3 planes), rows inverse (T -> F planes of a slice)
 void pass_rows_fwd(double* J, const TileGeom& tg, const FftPlan& p, cx* X, double* rl, double* rli, int i0, int j0,
                    int tr = 0);

@@ -631,7 +631,8 @@ __device__ __forceinline__ void stream_index(const StreamArgs& c, const Win& win
 // 512 x 386: 439 us with 2 waves, 528 capped for 4)
 constexpr int stream_waves(int YF, bool ION, bool LASER) { return YF == 1 && !ION && !LASER ? 4 : 1; }
 
-// workgroups 0 .. ntile-1: the particles of one tile with the LDS window, written to the tile's slab at the end;
+// workgroups 0 .. ntile-1: the particles of one tile with the LDS window, added to the current planes at the end (or,
+// without aflush, written to the tile's slab);
 // the following workgroups: the untiled particles from off[ntile] on, one per lane, global atomics
 // TILES: false for a list without tiles (the windows' code and registers left out).  Fourier y: a workgroup's deposits
 // are summed in an LDS box around its particles' midpoints, where they fit one (a list in the order of its lattice); the

@@ -1,6 +1,6 @@
 // One pass of a plasma half-cell after the particles, fused into three kernels around the transverse FFT:
 //
-//  k_pass_rows_fwd   the streaming current of the half-cell (jsr plus the tile slabs), the density lines,
+//  k_pass_rows_fwd   the streaming current of the half-cell (jsr, plus the tile slabs if there are), the density lines,
 //                    (j_x + i j_y, j_z) of a row -> x transform -> the pair unpacked per row (a real row has a
 //                    Hermitian x spectrum, so the unpack needs only the row itself); jsr is zeroed
 //  k_pass_cols       y transforms of the three planes of a block of columns in LDS, then per mode: the filters
