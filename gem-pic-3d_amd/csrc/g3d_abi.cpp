@@ -19,10 +19,10 @@ template <class T> size_t bytes_of(const DevBuf<T>& b) { return b.size() * sizeo
 
 // A large array to ordinary host memory: kReaders threads, each with two pinned buffers on the library's stream, copy one
 // chunk out while the next arrives.  The runtime's own copy to memory that is not pinned is serial and takes the page
-// faults of a new array in one thread: 1.6 GB, the fields at 256 x 256 x 1024, took about
-// 140 ms, now about 35; below kReadMin the pinning costs what it saves.  The buffers (32 MB) live for the call.  False when they or the
-// threads are not to be had; then nothing has been copied that a plain copy would not write again.
-constexpr size_t kReadChunk = size_t(2) << 20, kReadMin = size_t(32) << 20;
+// faults of a new array in one thread: 409 MB 38 -> 13 ms, 102 MB 9.7 -> 3.3, 51 MB 4.9 -> 1.8; at 34 MB 3.1 ms against
+// 1.4 to 3.8, hence kReadMin.  The buffers (32 MB) live for the call.  False when they or the threads are not to be had;
+// then nothing has been copied that a plain copy would not write again.
+constexpr size_t kReadChunk = size_t(2) << 20, kReadMin = size_t(48) << 20;
 constexpr int kReaders = 8;
 bool read_staged(char* host, const char* dev, size_t bytes) {
     struct Staging {

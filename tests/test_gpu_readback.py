@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 # F of 64 x 64 points: the last size of the plain copy, the first of the staged one (a few chunks more than the buffers'),
 # a long one with a short last chunk
-@pytest.mark.parametrize("nz", [339, 340, 1501])
+@pytest.mark.parametrize("nz", [509, 510, 1501])
 def test_large_array_round_trip(nz):
     d = g3d_amd.Deck(gi.LAMBDA0).grid(64, 64, nz, 64.0, 64.0, (nz - 1) * 0.5)
     d.set(dz=5.0, z_end=100.0, plasma_on=0)
