@@ -394,6 +394,11 @@ __global__ void __launch_bounds__(kDepLanes) k_dep_tile(DepositArgs c, const uns
     }
 }
 
+// Every buffer by its own length: the two sorts share some of them, and each needs other lengths of them
+template <class T> void fit(DevBuf<T>& b, long n) {
+    if (b.size() < size_t(n)) b.resize(size_t(n) + size_t(n) / 4);
+}
+
 // from which sizes the particle sort runs: whole tiles on a periodic grid, keys and records in 32 bits
 bool tiled_deposit(const DepositArgs& a, long np, unsigned& nbin) {
     if (!a.yf || a.nx % kDT || a.ny % kDT || a.nx < 2 * kDT || a.ny < 2 * kDT || np > (1L << 28)) return false;
@@ -407,14 +412,11 @@ void tiled_deposit_run(const DepositArgs& a, Parts p, long np, unsigned nbin, De
     const long n = np * kDepSlots;
     unsigned bits = 1;
     while ((1ull << bits) <= nbin) ++bits;            // the unused slots' key nbin among them
-    if (s.rec1.size() < size_t(n)) {
-        const size_t cap = size_t(n) + size_t(n) / 4;
-        s.k0.resize(cap); s.k1.resize(cap); s.rec1.resize(cap);
-    }
-    if (s.val.size() < size_t(kDepPack) * size_t(np)) s.val.resize(size_t(kDepPack) * size_t(np + np / 4));
+    fit(s.k0, n); fit(s.k1, n); fit(s.rec1, n);
+    fit(s.val, kDepPack * np);
     const int cap = int(std::min<long>(n, long(nbin)));
-    if (s.runs.size() < size_t(2) * size_t(cap)) s.runs.resize(size_t(2) * size_t(cap));
-    if (s.nruns.size() < 2) s.nruns.resize(2);
+    fit(s.runs, 2L * cap);
+    fit(s.nruns, 2);
     hipLaunchKernelGGL(k_dep_bins, dim3(blocks_for(np, kT)), dim3(kT), 0, stream(), a, p, np, ntx, nty, nbin, s.k0.data(),
                        s.val.data());
     size_t bytes = 0;
@@ -444,13 +446,8 @@ void bunch_deposit(const DepositArgs& a, Parts p, long np, DepositScratch& s) {
     int cb = 1;                                     // the bits of the cells hw nk + point
     while ((1ull << cb) < (unsigned long long)a.nh * (unsigned long long)a.nk) ++cb;
     if (cb > 60) throw std::runtime_error("beam deposit: grid too large");
-    if (s.key0.size() < size_t(n)) {
-        const size_t cap = size_t(n) + size_t(n) / 4;
-        s.key0.resize(cap); s.key1.resize(cap); s.rec0.resize(cap); s.rec1.resize(cap); s.val.resize(3 * cap);
-        s.vs.resize(3 * cap);
-    }
-    if (s.rec1.size() < size_t(n)) s.rec1.resize(s.key0.size());
-    if (s.val.size() < size_t(3 * n)) s.val.resize(3 * s.key0.size());
+    fit(s.key0, n); fit(s.key1, n); fit(s.rec0, n); fit(s.rec1, n);
+    fit(s.val, 3 * n); fit(s.vs, 3 * n);
     hipLaunchKernelGGL(k_dep_emit, dim3(blocks_for(np, kT)), dim3(kT), 0, stream(), a, p, np, R, cb, s.key0.data(),
                        s.rec0.data(), s.val.data());
     launch_check("beam deposit records");
@@ -467,8 +464,8 @@ void bunch_deposit(const DepositArgs& a, Parts p, long np, DepositScratch& s) {
                        s.val.data(), n, s.vs.data());
     // long runs: at most one per kShortRun + 1 records
     const int cap = int(n / (kShortRun + 1) + 1);
-    if (s.runs.size() < size_t(2 * cap)) s.runs.resize(size_t(2 * cap));
-    if (s.nruns.size() < 1) s.nruns.resize(1);
+    fit(s.runs, 2L * cap);
+    fit(s.nruns, 1);
     hip_check(hipMemsetAsync(s.nruns.data(), 0, sizeof(int), stream()), "hipMemsetAsync");
     hipLaunchKernelGGL(k_dep_sum, dim3(blocks_for(n, kT)), dim3(kT), 0, stream(), s.key1.data(), s.vs.data(), n, a.J,
                        long(a.nh), a.nk, a.yf, cb, s.runs.data(), s.nruns.data(), cap);

@@ -26,6 +26,17 @@ def stencil(x, d, n):
     (32, 32, 2, 20000, (16, 16), 1.6), (128, 64, 9, 30001, (100, 60), 40.0), (8, 16, 4, 700, (3, 3), 1.0),
     (4, 64, 4, 300, (2, 30), 3.0)])
 def test_deposit_order_and_spectra(nx, ny, ns, n, centre, sigma):
+    check(nx, ny, ns, n, centre, sigma)
+
+
+def test_both_sorts_on_the_same_buffers():
+    """the record sort (8 x 16 points) and the particle sort (32 x 32) in turn on the library's buffers, each call longer
+    than the other sort's buffers and, in the records they share, no longer than what the call before left"""
+    for nx, ny, n in ((8, 16, 40000), (32, 32, 100000), (8, 16, 120000), (32, 32, 300000)):
+        check(nx, ny, 4, n, (nx // 2, ny // 2), 2.0)
+
+
+def check(nx, ny, ns, n, centre, sigma):
     r = np.random.default_rng(n)
     dx, dy, h = 0.9, 0.7, 0.25
     p = np.zeros(n, dtype=g3d_amd.PARTICLE)
