@@ -36,9 +36,10 @@ public:
     }
     void resize(size_t n) {
         release();
-        n_ = n;
-        if (!n_) return;
-        hip_check(hipMalloc(reinterpret_cast<void**>(&p_), n_ * sizeof(T)), "hipMalloc");
+        if (!n) return;
+        T* p = nullptr;
+        hip_check(hipMalloc(reinterpret_cast<void**>(&p), n * sizeof(T)), "hipMalloc");
+        p_ = p; n_ = n;                  // only now: after a failed allocation the buffer is empty, not of size n
         zero();
     }
     void zero() { if (n_) hip_check(hipMemsetAsync(p_, 0, n_ * sizeof(T), stream()), "hipMemsetAsync"); }
