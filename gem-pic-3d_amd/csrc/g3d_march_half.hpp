@@ -25,7 +25,7 @@ struct Half6 { double Rx, Ry, Ez, Bz, Lx, Ly; };
 // corrected by its exact remainder, as the compiler's division does after its reciprocal, with div_fixup for infinities
 // and NaN.  Scaling is left out: den is at least 1 and x a field (a quotient below 1e-290 may differ in its last bit)
 struct HalfDen {
-    double h = -1, den = 1, r = 1;
+    double h = __builtin_nan(""), den = 1, r = 1;       // no step yet: NaN equals none
     __device__ __forceinline__ void set(const HalfK& k, double hn, double D) {
         if (hn == h) return;
         h = hn;

@@ -42,3 +42,36 @@ def test_staged_march_and_adjoint(monkeypatch, nx, ny, Lw):
     lhs, rhs = dot(w, out["1"]), dot(grads, old + cur)
     scale = math.sqrt(dot(w, w) * dot(out["1"], out["1"]))
     assert abs(lhs - rhs) <= 1e-13 * scale
+
+
+def arrays(geom, seed):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    mk = lambda rows: torch.randn(rows, geom.nk, dtype=torch.complex128, device="cuda", generator=g)
+    return mk
+
+
+def test_first_step_of_minus_one(monkeypatch):
+    """a march against zeta (D < 0) whose steps are -1 from the first slice on: the denominators are those of that step,
+    staged as plain, and the adjoint is the transpose"""
+    import torch
+    import g3d_autograd
+    sim = g3d_amd.Sim(march_deck(8, 4, 2.0))
+    geom = g3d_autograd.MarchGeometry(sim, -1.0)
+    geom.tables["hcg"].fill_(-1.0)
+    mk = arrays(geom, 5)
+    old, cur = [mk(geom.ns) for _ in range(4)], [mk(geom.ns + 1) for _ in range(5)]
+    out = {}
+    for staged in ("0", "1"):
+        monkeypatch.setenv("G3D_MARCH_STAGED", staged)
+        leaves = [t.clone().requires_grad_() for t in old + cur]
+        f = g3d_autograd.march(geom, leaves[:4], leaves[4:])
+        out[staged] = [t.detach() for t in f]
+    for a, b in zip(out["0"], out["1"]):
+        assert torch.isfinite(torch.view_as_real(a)).all() and torch.equal(a, b)
+    w = [mk(geom.ns) for _ in f]
+    grads = torch.autograd.grad(f, leaves, w)
+    dot = lambda a, b: sum(float((x.conj() * y).real.sum()) for x, y in zip(a, b))
+    # 10 slices of some 100 roundings of 1.1e-16 on either side
+    scale = math.sqrt(dot(w, w) * dot(out["1"], out["1"])) + math.sqrt(dot(grads, grads) * dot(old + cur, old + cur))
+    assert geom.ns == 10 and abs(dot(w, out["1"]) - dot(grads, old + cur)) <= 1e-13 * scale
