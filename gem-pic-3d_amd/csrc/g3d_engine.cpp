@@ -1468,7 +1468,7 @@ void Sim::march_plasma(double s0, double s1) {
         for (int k = 0; k < 4; ++k) {
             const bool on = k < int(cfg.ions.size()) && cfg.ions[k].ionization && nstrm > 0;
             ia.s[k] = IonStatSpecies{on ? ia.nslot : -1, on ? cfg.ions[k].Z0 : 0, on ? cfg.ions[k].Zmax : 0};
-            if (on) ia.nslot += cfg.ions[k].Zmax + 2;
+            if (on) ia.nslot += cfg.ions[k].Zmax + 3;
         }
         if (ia.nslot > 0) {
             if (ion_part.size() < size_t(kIonStatBlocks + 1) * ia.nslot) ion_part.resize(size_t(kIonStatBlocks + 1) * ia.nslot);
@@ -1476,8 +1476,11 @@ void Sim::march_plasma(double s0, double s1) {
             ion_statistics(ia, strmA.view(), nstrm, ion_part.data(), out);
             std::vector<double> v(static_cast<size_t>(ia.nslot));
             ion_part.to_host(v.data(), size_t(kIonStatBlocks) * ia.nslot, v.size());
-            for (size_t k = 0; k < ion_stats.size() && k < 4; ++k)
-                if (ia.s[k].slot >= 0) ion_stats[k].assign(v.begin() + ia.s[k].slot, v.begin() + ia.s[k].slot + ia.s[k].Zmax + 2);
+            for (size_t k = 0; k < ion_stats.size() && k < 4; ++k) {
+                if (ia.s[k].slot < 0) continue;
+                const auto h = v.begin() + ia.s[k].slot, e = h + ia.s[k].Zmax + 2;      // e: the number of its ions
+                if (*e > 0) ion_stats[k].assign(h, e);           // a species without an ion in the list: empty
+            }
         }
     }
     std::vector<g3d_particle> add;

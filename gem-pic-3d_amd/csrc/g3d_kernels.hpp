@@ -188,7 +188,8 @@ struct LatticeArgs {
 void plasma_lattice(const LatticeArgs& L, Parts A, Parts B, long ntile);
 // The ion statistics of a step (src/sim_plasma.cpp:438-446) summed on the device in a fixed tree order: for the
 // species of spec[0 .. nspec) (code SP_ION + k at slot[k] of out; slot -1: none) the weight of each charge state of
-// the ions still streaming, then the freed charge.  part: kIonStatBlocks nslot doubles of scratch
+// the ions still streaming, the freed charge, and the number of the species' ions in the list (any state): Zmax + 3
+// values.  part: kIonStatBlocks nslot doubles of scratch
 constexpr int kIonStatBlocks = 1024;
 struct IonStatSpecies { int slot, Z0, Zmax; };
 struct IonStatArgs { IonStatSpecies s[4]; int nslot; };

@@ -1120,6 +1120,7 @@ __global__ void __launch_bounds__(kIonStatLanes) k_ion_stats(IonStatArgs a, Part
         const double w = p.w[i];
         if (p.alive[i] == 1 && Z >= 0 && Z <= S.Zmax) ist[(S.slot + Z) * kIonStatLanes + t] += w;
         ist[(S.slot + S.Zmax + 1) * kIonStatLanes + t] += (Z - S.Z0) * w;
+        ist[(S.slot + S.Zmax + 2) * kIonStatLanes + t] += 1;
     }
     __syncthreads();
     for (int o = kIonStatLanes / 2; o > 0; o >>= 1) {

@@ -64,3 +64,21 @@ def test_ion_statistics_are_the_sums_of_the_list(yf, ny):
     want = [n["w"][(Z == z) & (n["alive"] == 1)].sum() for z in range(8)] + [(Z * n["w"]).sum()]
     assert want[8] > 0
     np.testing.assert_allclose(h, want, rtol=1e-12)
+
+
+def test_ion_statistics_of_a_species_without_ions_are_empty():
+    """a step outside the plasma with one electron waiting to join the stream: the list holds no ion, and the statistics of
+    an ionizing species are empty, not zeros"""
+    d = deck(1, 32, 32, (2, 1), "HN")
+    d.c.n_pz = 2
+    d.c.pz_points[0], d.c.pz_points[1] = 0.0, 100.0
+    d.c.pz_values[0], d.c.pz_values[1] = 0.0, 0.0
+    sim = g3d_amd.Sim(d)
+    sim.init()
+    p = np.zeros(1, dtype=g3d_amd.PARTICLE)
+    p["x"], p["y"], p["zeta"], p["z"] = 20.0, 15.0, 2.7, 0.0
+    p["w"], p["q"], p["qm"], p["alive"], p["sp"] = 1e-3, -1, -1, 1, 1
+    sim.set_joining(p)
+    sim.step()
+    assert sim.info()["nstrm"] == 1
+    assert len(sim.array("ion_stats0")) == 0 and len(sim.array("ion_stats1")) == 0
