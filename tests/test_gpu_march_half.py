@@ -1,4 +1,5 @@
 """The staged march and its adjoint (two real half-systems per mode) on grids and slice counts that leave remainders."""
+import ctypes as C
 import math
 
 import pytest
@@ -75,3 +76,45 @@ def test_first_step_of_minus_one(monkeypatch):
     # 10 slices of some 100 roundings of 1.1e-16 on either side
     scale = math.sqrt(dot(w, w) * dot(out["1"], out["1"])) + math.sqrt(dot(grads, grads) * dot(old + cur, old + cur))
     assert geom.ns == 10 and abs(dot(w, out["1"]) - dot(grads, old + cur)) <= 1e-13 * scale
+
+
+@pytest.mark.parametrize("nx,ny,cut", [(8, 4, 1), (16, 16, 4), (16, 16, 8), (8, 8, 7)])
+def test_window_in_two_parts(nx, ny, cut):
+    """the march of [cut, N) and then [0, cut), whose first slice takes slice cut as it stands, and the adjoint of [0, cut)
+    and then [cut, N) with `up` added to the adjoint of slice cut: bit for bit the calls over [0, N)"""
+    import torch
+    import g3d_autograd as ga
+    sim = g3d_amd.Sim(march_deck(nx, ny, 2.6))
+    geom = ga.MarchGeometry(sim, 2.5)
+    N, nk, lib = geom.N, geom.nk, g3d_amd.lib()
+    assert N % 6 and N % 3 and 0 < cut < N - 1
+    mk = arrays(geom, nx + cut)
+    fields, cur, bars, jbars = [mk(N) for _ in range(6)], [mk(N + 1) for _ in range(5)], [mk(N) for _ in range(6)], [mk(N + 1) for _ in range(5)]
+
+    def call(name, ctx, arrs, curs, parts, up=None):
+        a, b = [t.clone() for t in arrs], [t.clone() for t in curs]
+        c = ctx()
+        for n, t in list(zip(ga._FIELDS, a)) + list(zip(ga._CURRENTS, b)):
+            setattr(c, n, t.data_ptr())
+        geom._common(c)
+        if ctx is ga.MarchCtx:
+            c.b = N
+        for lo, hi in parts:
+            if ctx is ga.MarchAdjCtx:
+                c.up = up.data_ptr() if hi < N else None
+            torch.cuda.synchronize()
+            g3d_amd.check(getattr(lib, name)(C.byref(c), lo, hi))
+            g3d_amd.check(lib.g3d_sync())
+            if ctx is ga.MarchAdjCtx and hi < N:
+                for t, u in zip(a, up):
+                    t[hi] += u
+        return a + b
+
+    for got, want in zip(call("g3d_march", ga.MarchCtx, fields, cur, [(cut, N), (0, cut)]),
+                         call("g3d_march", ga.MarchCtx, fields, cur, [(0, N)])):
+        assert torch.equal(got, want)
+    up = torch.zeros(6, nk, dtype=torch.complex128, device="cuda")
+    for got, want in zip(call("g3d_march_adjoint", ga.MarchAdjCtx, bars, jbars, [(0, cut), (cut, N)], up),
+                         call("g3d_march_adjoint", ga.MarchAdjCtx, bars, jbars, [(0, N)])):
+        assert torch.equal(got, want)
+    assert up.abs().max() > 0
