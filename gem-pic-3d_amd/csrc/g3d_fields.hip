@@ -350,6 +350,7 @@ void currents_unpack(const SpecGeom& g, const cx* S1, cx* jkx, cx* jky, cx* jkz,
 }
 void sponge_pack(const SpecGeom& g, const cx* Rx, const cx* Ry, const cx* jkz, const double* hcg, const double* wlo,
                  const double* whi, double g2, double opb, cx* S1, cx* S2) {
+    if (g.cm) throw std::runtime_error("sponge: row-major modes only");
     G3D_LAUNCH(k_sponge_pack, long(g.ns) * g.nk, g, Rx, Ry, jkz, hcg, wlo, whi, g2, opb, S1, S2);
 }
 void sponge_mask(const SpecGeom& g, cx* S1, const double* mx, const double* mn, const double* mh, int count) {
@@ -357,6 +358,7 @@ void sponge_mask(const SpecGeom& g, cx* S1, const double* mx, const double* mn, 
 }
 void fields_pack3(const SpecGeom& g, const cx* S1, const cx* S2, double opb, cx* Rx, cx* Ry, const cx* Lx,
                   const cx* Ly, const cx* Ez, const cx* Bz, cx* T, long ts, int count) {
+    if (g.cm) throw std::runtime_error("pack: row-major modes only");
     G3D_LAUNCH(k_pack3, long(count) * g.nk, g, S1, S2, opb, Rx, Ry, Lx, Ly, Ez, Bz, T, ts, long(count) * g.nk);
 }
 void fields_to_F(const cx* T, long ts, float* F, long fpl, long nk, int count) {
