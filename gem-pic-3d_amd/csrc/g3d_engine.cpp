@@ -1443,7 +1443,8 @@ void Sim::march_plasma(double s0, double s1) {
     std::vector<g3d_particle> sv;
     {
         counters.zero();
-        if (aos.size() < std::max<size_t>(strmA.cap, 1)) aos.resize(std::max<size_t>(strmA.cap, 1));
+        // the list as it is now, not its capacity (which holds every electron that the ions could free)
+        if (aos.size() < size_t(std::max<long>(nstrm, 1))) aos.resize(size_t(nstrm + nstrm / 4 + 1));
         if (aos_idx.size() < aos.size()) aos_idx.resize(aos.size());
         collect_alive(strmA.view(), nstrm, 5, aos.data(), aos_idx.data(), counters.data() + 1, long(aos.size()));
         int cnt = 0;

@@ -69,3 +69,22 @@ def test_mixed_witness_energy_gain():
     assert abs(gain64) > 1e-3, "the witness must gain or lose energy"
     assert rel <= GAIN_TOL, rel
     assert err["fields"] <= FIELD_TOL, err
+
+
+@pytest.mark.parametrize("mixed", [0, 1])
+def test_windows_through_slabs(monkeypatch, mixed):
+    """the tiles' current windows through slabs (made in the step that wants them) against windows added to the planes: the
+    same sums in another order, in FP64 to the parity bar, in FP32 to the mixed form's"""
+    out = []
+    for aflush in ("11", "01", "10"):           # the switch is looked at in every step
+        d = plasma_deck(a0=2.0)
+        d.set(mixed=mixed)
+        sim = g3d_amd.Sim(d)
+        sim.init()
+        for e in aflush:
+            monkeypatch.setenv("G3D_STREAM_AFLUSH", e)
+            sim.step()
+        out.append([sim.array(n) for n in SPEC])
+    ns = sim.info()["ns"]
+    for o in out[1:]:
+        assert group_rel_l2(o, out[0], ns) <= (FIELD_TOL if mixed else 1e-12)
