@@ -270,8 +270,7 @@ void Sim::setup_tiles() {
     tiles.fh = !yf;
     tiles.fy = yax;
     tile_off.resize(tiles.ntile + 1);
-    slab.resize(size_t(tiles.ntile) * 5 * tiles.WX * tiles.WY);
-    tiles.off = tile_off.data(); tiles.slab = slab.data(); tiles.n_tiled = 0;
+    tiles.off = tile_off.data(); tiles.slab = nullptr; tiles.n_tiled = 0;
     const char* e = getenv("G3D_STREAM_FWIN");
     tiles.fwin = e ? atoi(e) : 1;
     // lanes per tile workgroup (about the particles of a tile; free-hand y with its ions: 256, 2 % faster than 512
@@ -1241,7 +1240,7 @@ void Sim::march_plasma(double s0, double s1) {
     };
     StreamArgs sc = stream_args(s0, s1);
     const bool ionz = born_cap > 0;
-    // tiles only when this step loaded tiled plasma (otherwise the slabs would hold an earlier step's current)
+    // tiles only when this step loaded tiled plasma (tile_off and slabs are an earlier step's otherwise)
     TileGeom tg = n_tiled > 0 ? tiles : TileGeom{};
     tg.idx = nullptr;
     tg.chunk = 0; tg.max_extra = 0; tg.xtile = nullptr; tg.xstart = nullptr; tg.xcount = nullptr;
@@ -1251,8 +1250,14 @@ void Sim::march_plasma(double s0, double s1) {
     // the tile windows go to the current planes with atomics instead of slabs: the row kernel then reads one plane set.
     // FP32-mixed: 3 % of a step at 256 x 256; FP64, 4 a cell: rows 8.1 -> 4.5 us against 14.2 -> 14.7 of the stream at
     // 64 x 64, 8.6 -> 4.9 against 15.4 -> 16.0 at 128 x 128, 10.1 -> 6.5 against 27.5 -> 28.7 at 256 x 256.
-    // G3D_STREAM_AFLUSH=0 keeps the slabs
+    // G3D_STREAM_AFLUSH=0: slabs, which exist only then
     { const char* e = getenv("G3D_STREAM_AFLUSH"); tg.aflush = !(e && atoi(e) == 0) || mxi; }
+    if (tg.ntile && !tg.aflush && yf) {
+        const size_t n = size_t(tg.ntile) * 5 * tg.WX * tg.WY;
+        if (mx && slab_f.size() < n) slab_f.resize(n);
+        if (!mx && slab.size() < n) slab.resize(n);
+        tg.slab = slab.data();
+    }
     // FP32-mixed: tiles denser than G3D_STREAM_CHUNK (default 1) times one workgroup's lanes are streamed in
     // chunks of that many particles (0: off)
     const char* ech = getenv("G3D_STREAM_CHUNK");
@@ -1272,11 +1277,7 @@ void Sim::march_plasma(double s0, double s1) {
         if (jsr_f.size() < 5 * pl) jsr_f.resize(5 * pl);
         sc.Jf = jsr_f.data();
     }
-    if (mx) {
-        if (jsr_f.size() < 5 * pl) jsr_f.resize(5 * pl);
-        if (tiles.ntile && slab_f.size() < size_t(tiles.ntile) * 5 * tiles.WX * tiles.WY)
-            slab_f.resize(size_t(tiles.ntile) * 5 * tiles.WX * tiles.WY);
-    }
+    if (mx && jsr_f.size() < 5 * pl) jsr_f.resize(5 * pl);
     // the stream launches count their pushes per workgroup: at most every tile, every further chunk and the
     // untiled rest of the list in workgroups of at least 64 lanes
     const long npc = tg.ntile + tg.max_extra + (long(strmA.cap) + 63) / 64 + 1;
