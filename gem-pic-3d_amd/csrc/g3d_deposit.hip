@@ -19,8 +19,8 @@
 //
 // On a periodic grid of whole 8 x 8 tiles (k_dep_tile) the sort is of particles instead of their 9 records: a particle
 // is listed in every (half-cell, tile) bin that its stencil touches (at most 4, 1.6 on average), and a workgroup per bin
-// adds the records of its 64 cells in particle order from LDS.  2^20 electrons in 128 slices of 256 x 256: 1.45 -> 0.48 ms
-// (bins 53 us, sort 130, tiles 283); 2^18 in 256 of 64 x 64: 0.44 -> 0.22 ms.
+// (a wave, for a bin of few: k_dep_wave) adds the records of its 64 cells in particle order.  2^20 electrons in 128 slices
+// of 256 x 256: 1.45 -> 0.49 ms (bins 53 us, sort 130, tiles 283); 2^18 in 256 of 64 x 64: 0.44 -> 0.23 ms.
 #include <algorithm>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -32,8 +32,10 @@
 namespace g3d {
 namespace {
 constexpr int kT = 256;
-// radix passes at every length: the default sorts up to 2^20 records by merging, a score of launches (140 us for 2^20)
+// Long lists by radix passes: the default merges up to 2^20 records, a score of launches.  g3d_bunch_currents with keys of 15
+// bits, radix and merged: 4000 keys 133 and 94 us, 16384 152 and 113, 65536 157 and 128, 2^18 170 and 195
 using DepSort = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config, rocprim::default_config, 0>;
+constexpr long kMergeSort = 1L << 17;                // keys up to which the default is used
 constexpr unsigned long long kNone = ~0ull;
 // key of a record: cell = hw nk + point in the low cb bits (cb: the bits of nh nk), the half-node group in bit cb;
 // the sort looks at bits 0 .. cb+1 only, where the empty key ~0 has all ones and so follows every cell
@@ -205,13 +207,15 @@ constexpr int kDepSlots = 4;                         // tiles that a 3 x 3 stenc
 constexpr int kDepLanes = 512;                       // particles of a chunk
 constexpr int kDepWaves = kDepLanes / 64;
 constexpr int kDepLong = 512;                        // bins of more particles are taken first
+constexpr int kDepFew = 32;                          // bins of at most that many: a wave each (k_dep_wave)
 constexpr int kDepPack = 8;                          // doubles per packed particle: xi, yi, f, v_x, v_y, v_z, -, -
 
 // the bins of every particle (slot order = particle order; unused slots: nbin) and what the tiles need of it in one
-// 64-byte record (a bin's particles lie anywhere in the list)
+// 64-byte record (a bin's particles lie anywhere in the list); the counts of k_dep_runs are cleared on the way
 __global__ void __launch_bounds__(kT) k_dep_bins(DepositArgs c, Parts P, long np, int ntx, int nty, unsigned nbin,
-                                                 unsigned* key, double* pack) {
+                                                 unsigned* key, double* pack, int* cnt) {
     const long ip = long(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (ip < 3) cnt[ip] = 0;
     if (ip >= np) return;
     unsigned k[kDepSlots] = {nbin, nbin, nbin, nbin};
     int m = 0; double fz;
@@ -244,7 +248,8 @@ __global__ void __launch_bounds__(kT) k_dep_bins(DepositArgs c, Parts P, long np
     }
     *reinterpret_cast<uint4*>(key + kDepSlots * ip) = make_uint4(k[0], k[1], k[2], k[3]);
 }
-// the runs of equal keys: (first record, end) of the long ones from the front of `bins`, of the others from its back
+// the runs of equal keys, (first record, end) each: in the first `cap` slots of `bins` the long ones from the front and
+// those of more than kDepFew records from the back, from slot cap on the others (cnt: the three numbers)
 __global__ void __launch_bounds__(kT) k_dep_runs(const unsigned* key, long n, unsigned nbin, long* bins, int* cnt, int cap) {
     const long i = long(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -261,9 +266,11 @@ __global__ void __launch_bounds__(kT) k_dep_runs(const unsigned* key, long n, un
         const long mid = lo + ((hi - lo) >> 1);
         if (key[mid] == k) lo = mid + 1; else hi = mid;
     }
-    const bool lng = lo - i > kDepLong;
-    const int r = atomicAdd(&cnt[lng ? 0 : 1], 1);
-    const long slot = lng ? r : long(cap) - 1 - r;          // every run has its slot: runs <= cap
+    // every run has its slot: runs <= cap.  One address per branch: the compiler then adds once per wave
+    long slot;
+    if (lo - i > kDepLong) slot = atomicAdd(&cnt[0], 1);
+    else if (lo - i > kDepFew) slot = long(cap) - 1 - atomicAdd(&cnt[1], 1);
+    else slot = long(cap) + atomicAdd(&cnt[2], 1);
     bins[2 * slot] = i; bins[2 * slot + 1] = lo;
 }
 // x / d with r = 1 / d: the quotient estimate and one exact correction, as the compiler's division ends, with div_fixup for
@@ -394,6 +401,68 @@ __global__ void __launch_bounds__(kDepLanes) k_dep_tile(DepositArgs c, const uns
     }
 }
 
+// The bins of few particles, a wave each: the particles' stencils formed by a lane each and left in LDS, then one lane per
+// cell of the tile takes the particles in list order (a chain of kDepFew records, about a chunk of k_dep_tile).  That
+// kernel's workgroup fills a CU with its lists, so it takes 256 bins at a time however few their particles: electrons
+// anywhere in 128 slices of 16 x 512 points, all of g3d_bunch_currents, with the tiles alone, now, and by the record sort
+// (8 x 1024 points): 16384 electrons 441, 125 and 168 us; 65536 538, 178 and 288; 2^18 565, 292 and 440; 10^5 in 256 x 256
+// 2580 and 590.  A bunch pays a launch: 65536 166 -> 170 us, 2^18 233 -> 237.  kDepFew 16: 2^18 anywhere 453 us; 64:
+// 268, but the bunches 174 and 241.
+constexpr int kFewWaves = 4;                         // bins of a workgroup at a time
+constexpr int kFewRec = 11;                          // doubles per particle: f w_x (3), w_y (3), v_x, v_y, v_z, 1/v_z, first nodes
+__global__ void __launch_bounds__(64 * kFewWaves) k_dep_wave(DepositArgs c, const unsigned* key, const unsigned* rec,
+                                                             const double* pack, const long* bins, const int* cnt, int cap,
+                                                             int ntx, int nty) {
+    __shared__ double buf[kFewWaves][kDepFew * kFewRec];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    double* B = buf[wv];
+    const int nb = cnt[2];
+    for (int b = blockIdx.x * kFewWaves + wv; b < nb; b += gridDim.x * kFewWaves) {
+        const long lo = bins[2 * (long(cap) + b)];
+        const int m = int(bins[2 * (long(cap) + b) + 1] - lo);
+        const unsigned k = key[lo];
+        const int tile = int(k % unsigned(ntx * nty)), hw = int(k / unsigned(ntx * nty));
+        const int x0 = (tile % ntx) * kDT, y0 = (tile / ntx) * kDT;
+        if (lane < m) {
+            const double2* q = reinterpret_cast<const double2*>(pack + kDepPack * long(rec[lo + lane] / kDepSlots));
+            const double2 q0 = q[0], q1 = q[1], q2 = q[2];
+            int ix[3], jn[3]; double wx[3], wn[3];
+            tsc_w(q0.x, ix, wx);
+            tsc_w(q0.y, jn, wn);
+            double* r = B + kFewRec * lane;
+#pragma unroll
+            for (int u = 0; u < 3; ++u) { r[u] = q1.x * wx[u]; r[3 + u] = wn[u]; }
+            r[6] = q1.y; r[7] = q2.x; r[8] = q2.y; r[9] = 1 / q2.y;
+            reinterpret_cast<int2*>(r + 10)[0] = make_int2(wrap_index(ix[0], c.nx), wrap_index(jn[0], c.ny));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int x = x0 + (lane & (kDT - 1)), y = y0 + lane / kDT;
+        double a0 = 0, a1 = 0, a2 = 0;
+        // no branch: a particle that misses the cell adds zero, which never changes a sum that began as +0
+#pragma unroll 4
+        for (int t = 0; t < m; ++t) {
+            const double* r = B + kFewRec * t;
+            const int2 n0 = reinterpret_cast<const int2*>(r + 10)[0];
+            int u = x - n0.x, v = y - n0.y;
+            u += u < 0 ? c.nx : 0;
+            v += v < 0 ? c.ny : 0;
+            const bool in = u < 3 && v < 3;
+            const double w = r[in ? u : 0] * r[3 + (in ? v : 0)] * c.ia[0], vz = r[8], rz = r[9];
+            const double p0 = div_by(w * r[6], vz, rz), p1 = div_by(w * r[7], vz, rz);
+            a0 += in ? p0 : 0.0;
+            a1 += in ? p1 : 0.0;
+            a2 += in ? w : 0.0;
+        }
+        double* J = c.J + long(hw) * c.nk + long(y) * c.nx + x;
+        const long pl = long(c.nh) * c.nk;
+        J[0] = a0; J[pl] = a1; J[2 * pl] = a2;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();              // before the next bin's records
+    }
+}
+
 // Every buffer by its own length: the two sorts share some of them, and each needs other lengths of them
 template <class T> void fit(DevBuf<T>& b, long n) {
     if (b.size() < size_t(n)) b.resize(size_t(n) + size_t(n) / 4);
@@ -415,23 +484,28 @@ void tiled_deposit_run(const DepositArgs& a, Parts p, long np, unsigned nbin, De
     fit(s.k0, n); fit(s.k1, n); fit(s.rec1, n);
     fit(s.val, kDepPack * np);
     const int cap = int(std::min<long>(n, long(nbin)));
-    fit(s.runs, 2L * cap);
-    fit(s.nruns, 2);
+    fit(s.runs, 4L * cap);
+    fit(s.nruns, 3);
     hipLaunchKernelGGL(k_dep_bins, dim3(blocks_for(np, kT)), dim3(kT), 0, stream(), a, p, np, ntx, nty, nbin, s.k0.data(),
-                       s.val.data());
-    size_t bytes = 0;
+                       s.val.data(), s.nruns.data());
     const rocprim::counting_iterator<unsigned> ids(0);
-    hip_check(rocprim::radix_sort_pairs<DepSort>(nullptr, bytes, s.k0.data(), s.k1.data(), ids, s.rec1.data(), n, 0, bits, stream()),
-              "beam deposit sort size");
-    if (s.tmp.size() < bytes) s.tmp.resize(bytes + bytes / 4 + 256);
-    bytes = s.tmp.size();
-    hip_check(rocprim::radix_sort_pairs<DepSort>(s.tmp.data(), bytes, s.k0.data(), s.k1.data(), ids, s.rec1.data(), n, 0, bits,
-                                        stream()), "beam deposit sort");
-    hip_check(hipMemsetAsync(s.nruns.data(), 0, 2 * sizeof(int), stream()), "hipMemsetAsync");
+    auto sort = [&](auto config) {
+        size_t bytes = 0;
+        hip_check(rocprim::radix_sort_pairs<decltype(config)>(nullptr, bytes, s.k0.data(), s.k1.data(), ids, s.rec1.data(), n, 0, bits,
+                                                              stream()), "beam deposit sort size");
+        if (s.tmp.size() < bytes) s.tmp.resize(bytes + bytes / 4 + 256);
+        bytes = s.tmp.size();
+        hip_check(rocprim::radix_sort_pairs<decltype(config)>(s.tmp.data(), bytes, s.k0.data(), s.k1.data(), ids, s.rec1.data(), n, 0,
+                                                              bits, stream()), "beam deposit sort");
+    };
+    if (n <= kMergeSort) sort(rocprim::default_config{});
+    else sort(DepSort{});
     hipLaunchKernelGGL(k_dep_runs, dim3(blocks_for(n, kT)), dim3(kT), 0, stream(), s.k1.data(), n, nbin, s.runs.data(),
                        s.nruns.data(), cap);
     hipLaunchKernelGGL(k_dep_tile, dim3(unsigned(std::min(cap, 1024))), dim3(kDepLanes), 0, stream(), a, s.k1.data(),
                        s.rec1.data(), s.val.data(), s.runs.data(), s.nruns.data(), cap, ntx, nty);
+    hipLaunchKernelGGL(k_dep_wave, dim3(std::min(blocks_for(cap, kFewWaves), 2048u)), dim3(64 * kFewWaves), 0, stream(), a,
+                       s.k1.data(), s.rec1.data(), s.val.data(), s.runs.data(), s.nruns.data(), cap, ntx, nty);
     launch_check("beam deposit (tiles)");
 }
 }  // namespace

@@ -29,6 +29,15 @@ def test_deposit_order_and_spectra(nx, ny, ns, n, centre, sigma):
     check(nx, ny, ns, n, centre, sigma)
 
 
+# a bin of exactly 32 particles (the last that a wave takes), of 33, of 512 (the last of one chunk), of 513; particles all
+# over a window (nearly all bins of few); the longest list whose keys are merged, and one particle more
+@pytest.mark.parametrize("nx,ny,ns,n,centre,sigma", [
+(16, 16, 2, 39, (8, 8), 0.0), (16, 16, 3, 67, (8, 8), 0.0), (16, 16, 2, 604, (8, 8), 0.0), (16, 16, 3, 1107, (8, 8), 0.0),
+    (32, 64, 20, 6000, (16, 32), 30.0), (32, 32, 6, 32768, (16, 16), 3.0), (32, 32, 6, 32769, (16, 16), 3.0)])
+def test_deposit_of_few_and_many(nx, ny, ns, n, centre, sigma):
+    check(nx, ny, ns, n, centre, sigma)
+
+
 def test_both_sorts_on_the_same_buffers():
     """the record sort (8 x 16 points) and the particle sort (32 x 32) in turn on the library's buffers, each call longer
     than the other sort's buffers and, in the records they share, no longer than what the call before left"""
