@@ -96,12 +96,14 @@ bool tile_index_fit(TileIndex& t, long n, long ntile) {
     return ok;
 }
 // Whether a half-cell is streamed through tiles, which costs three launches for the index.  With the spectra of the
-// current, untiled (a workgroup's deposits summed in its box) and tiled, in us: lists in the order of their lattice
-// 6.6 x 10^4 particles at 4 per cell 30 and 44, 1.3 x 10^5 at 4 per cell 44 and 50, 2.0 x 10^5 at 3 per cell 53 and 61,
-// 2.6 x 10^5 at 4 per cell 65 and 67, 3.9 x 10^5 at 6 per cell 84 and 86; a list in no order keeps the tiled times but,
-// untiled, takes those of one atomic per deposit (290 for 2.6 x 10^5).  So from the length on where the order no longer
-// matters for the better.  Periodic grids that hold the tiles, with both field slices present.  The results are the
-// untiled kernel's but for the order of the current's sums, which its atomics leave free as well
+// current on 256 x 256 points, untiled (a workgroup's deposits summed in its box) and tiled, in us: lists in the order of
+// their lattice 6.6 x 10^4 particles 41 and 50, 1.3 x 10^5 48 and 56, 2.0 x 10^5 52 and 62, 2.6 x 10^5 60 and 71,
+// 3.9 x 10^5 79 and 94; the same numbers anywhere 152 and 64, 277 and 92, 375 and 120, 471 and 153, 679 and 208.  A list in
+// its lattice's order is never better off with tiles (by 15 to 20 % here; by more where few tiles hold many particles: 64 x 64
+// points with 64 per cell 81 and 275), one in no order always is: the tiles are the insurance of the long lists, whose order
+// is not known here and whose loss without them is the largest.  Periodic grids that hold the tiles, with both field slices
+// present.  The results are the untiled kernel's but for the order of the current's sums, which its atomics leave free as
+// well
 constexpr long kTiledMin = 200000;
 bool tiled_halfcell(const StreamArgs& a, long n, TileGeom& tg) {
     const FieldView& F = a.fv;

@@ -638,7 +638,7 @@ constexpr int stream_waves(int YF, bool ION, bool LASER) { return YF == 1 && !IO
 // are summed in an LDS box around its particles' midpoints, where they fit one (a list in the order of its lattice); the
 // deposits that miss the box, or find none, take the global atomics, 36 per particle, which bounded the kernel.  With the
 // spectra of the current: 8.2 x 10^3 electrons at 2 per cell 31 -> 23 us, 3.3 x 10^4 at 2 per cell 49 -> 26, 2.0 x 10^5
-// at 3 per cell 216 -> 50; 4.1 x 10^3 at 1 per cell 25 -> 23 (a chain of loads and FP64 operations of one wave, 15 us)
+// at 3 per cell 216 -> 52; 4.1 x 10^3 at 1 per cell 25 -> 23 (a chain of loads and FP64 operations of one wave, 15 us)
 constexpr int kBoxNodes = 8;          // the largest box, per lane: 5 planes of 8 nodes, 20 KB for 64 lanes
 template <int YF, bool ION, bool LASER, bool TILES>
 __global__ void __launch_bounds__(kStreamBlockMax)
