@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 
 import g3d_amd
+import oraclepy as orc
 import refpy
 
 pytestmark = pytest.mark.gpu
@@ -267,11 +268,10 @@ IP = {"H": [13.598434599702], "N": [14.53413, 29.60125, 47.4453, 77.4735, 97.890
 MASS_U = {"H": 1.00794, "N": 14.0067}
 
 
-def ionization_run(el, Z0, Zmax, mobile, a0):
+def ionization_run(el, Z0, Zmax, mobile, a0, rate=None):
     """tests/test_ionization.cpp:38-82: atoms at 1e-6 n_c loaded at the front of the window, the analytic
     s-polarised plane-wave pulse (c tau = 30/k0, lambda0 = 0.8 um) centred in the window; after one step the
     fractions of the charge states against the rate equations along the path of an atom at rest"""
-    import refpy
     tau = 30.0
     h = 2 * math.pi / 40
     N = int(6 * tau / h) + 1
@@ -304,7 +304,7 @@ def ionization_run(el, Z0, Zmax, mobile, a0):
     dt, eps = h / 50, 1e-4
     ets = np.arange(-(Lw - 0.5 * Lw), 0.5 * Lw, dt)
     es = np.abs(-(A(ets + 0.5 * dt + eps) - A(ets + 0.5 * dt - eps)) / (2 * eps)) * E0
-    rate = refpy.lib().ref_adk_rate_SI          # the reference's ADK rate in SI (checked against Landau's form)
+    rate = rate or refpy.lib().ref_adk_rate_SI   # the reference's ADK rate in SI (checked against Landau's form)
     for e in es:
         w = [rate(IP[el][k], k + 1, float(e)) * dt / omega0 for k in range(Z0, Zmax)]
         if Zmax - Z0 == 1:
@@ -329,6 +329,27 @@ def test_field_ionization_rate_equations():
     f, ref = ionization_run("H", 0, 1, False, 0.01)
     close(f[1], ref[1], 0.03, "H ionized fraction (fixed atoms, a0 = 0.01)")
     f, ref = ionization_run("N", 5, 7, True, 2.0)
+    close(f[0], ref[0], 0.05, "N5+ fraction after the pulse (a0 = 2)")
+    close(f[1], ref[1], 0.03, "N6+ fraction after the pulse")
+    close(f[2], ref[2], 0.10, "N7+ fraction after the pulse")
+
+
+@pytest.mark.skipif(not orc.available(), reason="oracle not built")
+def test_field_ionization_rate_equations_by_the_oracle():
+    """the same with the ADK rate of the oracle, which tests/test_oracle.py holds to the reference's levels and to Landau's
+    form"""
+    omega0 = 299792458.0 / (0.8e-6 / (2 * math.pi))
+    E0 = 9.1093837015e-31 * 299792458.0 * omega0 / 1.602176634e-19
+
+    def rate(U, Z, E):
+        ip = np.zeros(Z)
+        ip[Z - 1] = U
+        lev = orc.adk_levels(ip, Z - 1, Z, E0, omega0, 1e4)[Z - 1]      # no rate below 1e-10 over 10^4 / omega0
+        return orc.adk_rate(lev, E / E0) * omega0
+
+    f, ref = ionization_run("H", 0, 1, False, 0.01, rate)
+    close(f[1], ref[1], 0.03, "H ionized fraction (fixed atoms, a0 = 0.01)")
+    f, ref = ionization_run("N", 5, 7, True, 2.0, rate)
     close(f[0], ref[0], 0.05, "N5+ fraction after the pulse (a0 = 2)")
     close(f[1], ref[1], 0.03, "N6+ fraction after the pulse")
     close(f[2], ref[2], 0.10, "N7+ fraction after the pulse")
