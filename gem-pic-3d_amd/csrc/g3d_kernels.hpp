@@ -121,7 +121,8 @@ struct DepositScratch {
 // the reference's single-thread summation order, bit for bit (g3d_deposit.hip)
 void bunch_deposit(const DepositArgs& a, Parts p, long np, DepositScratch& s);
 // one half-cell pass of the streaming particles: src -> dst (the state of every particle is written); tiles
-// with tg.ntile > 0, otherwise every deposit is a global atomic
+// with tg.ntile > 0; otherwise Fourier y: a workgroup's deposits summed in a box where they fit one, free-hand y: every
+// deposit a global atomic
 // start and stop events of one launch, recorded by the launch itself (no marker packets around it); null: untimed
 struct LaunchTimer {
     hipEvent_t start = nullptr, stop = nullptr;
