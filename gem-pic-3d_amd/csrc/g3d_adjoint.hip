@@ -21,7 +21,8 @@ namespace {
 // Slices lo ... hi-1 of every mode, rear to front: the transpose of the march.  Like k_march_staged, two lanes per
 // mode (one real half-system each) and 32 modes per workgroup: wave 0 runs the chain from LDS, waves 1-3 load the next
 // block of kAdjB slices (one each) into the other of two buffers and clear L_x, L_y, which are not inputs.  As one
-// lane per mode with complex arithmetic and its loads on the chain it took 742 us for 64 x 64 x 256, now 141 us.
+// lane per mode with complex arithmetic and its loads on the chain it took 742 us for 64 x 64 x 256, now 143 us.  Larger grids
+// are bound by the 22 planes that a slice reads and writes: 256 x 256 x 64 298 us, 512 x 512 x 32 646 us (5.0 and 4.6 TB/s).
 constexpr int kAdjB = 3, kAdjComp = 11;
 __global__ void __launch_bounds__(256) k_march_adj(AdjView c, int lo, int hi) {
     __shared__ double stg[2 * kAdjB * kAdjComp * 64], wts[2 * kAdjB * 3];

@@ -42,9 +42,10 @@ __device__ __forceinline__ void tsc_wd(double x, double d, int n, int idx[3], do
 // ---------------------------------------------------------------- sums of a workgroup's neighbouring particles in LDS
 // (node_box): one global atomic per node and plane of the box of kBoxT consecutive particles.  With one per contribution
 // (108 per particle of the reverse, 36 of the push) these bound both kernels, at 34 x 10^9 atomics a second: 32768
-// particles on 128 x 128 nodes took 105 us and 36 us, now 67 us and 16 us, and 8192 on 64 x 64 in the reverse 31 us, now
+// particles on 128 x 128 nodes took 105 us and 36 us, now 30 us and 14 us, and 8192 on 64 x 64 in the reverse 31 us, now
 // 25 us (there the chain of a particle's operations bounds it).  128 lanes: 64 hold half the particles a node, and 256
-// leave half of the CUs idle at these sizes.  A box beyond the LDS (a list in no order) takes the global atomics.
+// leave half of the CUs idle at these sizes.  A box beyond the LDS (a list in no order) takes the global atomics,
+// no slower than workgroups of 256 without the box.
 constexpr int kBoxT = 128;
 // the workgroup's particles
 __device__ __forceinline__ int box_lanes(const g3d_spush_ctx& c) {
