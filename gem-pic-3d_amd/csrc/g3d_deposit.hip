@@ -19,8 +19,8 @@
 //
 // On a periodic grid of whole 8 x 8 tiles (k_dep_tile) the sort is of particles instead of their 9 records: a particle
 // is listed in every (half-cell, tile) bin that its stencil touches (at most 4, 1.6 on average), and a workgroup per bin
-// (a wave, for a bin of few: k_dep_wave) adds the records of its 64 cells in particle order.  2^20 electrons in 128 slices
-// of 256 x 256: 1.45 -> 0.49 ms (bins 53 us, sort 130, tiles 283); 2^18 in 256 of 64 x 64: 0.44 -> 0.23 ms.
+// (a wave, for a bin of few) adds the records of its 64 cells in particle order.  2^20 electrons in 128 slices of
+// 256 x 256: 1.45 -> 0.48 ms (bins 55 us, sort 130, tiles 282); 2^18 in 256 of 64 x 64: 0.44 -> 0.22 ms.
 #include <algorithm>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -207,7 +207,7 @@ constexpr int kDepSlots = 4;                         // tiles that a 3 x 3 stenc
 constexpr int kDepLanes = 512;                       // particles of a chunk
 constexpr int kDepWaves = kDepLanes / 64;
 constexpr int kDepLong = 512;                        // bins of more particles are taken first
-constexpr int kDepFew = 32;                          // bins of at most that many: a wave each (k_dep_wave)
+constexpr int kDepFew = 32;                          // bins of at most that many: a wave each (dep_few)
 constexpr int kDepPack = 8;                          // doubles per packed particle: xi, yi, f, v_x, v_y, v_z, -, -
 
 // the bins of every particle (slot order = particle order; unused slots: nbin) and what the tiles need of it in one
@@ -279,7 +279,61 @@ __device__ __forceinline__ double div_by(double x, double d, double r) {
     const double q = x * r;
     return __builtin_amdgcn_div_fixup(fma(fma(-q, d, x), r, q), d, x);
 }
-// One workgroup per bin (persistent).  A chunk of kDepLanes particles at a time, in list order: which of the tile's 8
+constexpr int kFewRec = 11;                          // doubles per particle: f w_x (3), w_y (3), v_x, v_y, v_z, 1/v_z, first nodes
+// A bin of at most kDepFew particles by one wave, B: kDepFew records of LDS: the particles' stencils formed by a lane each
+// and left there, then one lane per cell of the tile takes the particles in list order.  A workgroup of k_dep_tile fills a CU
+// with its lists, so 256 bins went through at a time however few their particles.  Electrons anywhere in 128 slices of 16 x 512
+// points, all of g3d_bunch_currents, with a workgroup for every bin, now, and by the record sort (8 x 1024 points): 16384
+// electrons 441, 130 and 168 us; 65536 538, 187 and 288; 2^18 565, 304 and 440; 10^5 in 256 x 256 2580 and 610.  In a launch
+// of their own the small bins take up to 20 us less there, but bunches pay for it (65536 171 us, here 167); so launched,
+// kDepFew 16, 32 and 64: 2^18 anywhere 453, 293 and 268 us, a bunch of 2^18 236, 237 and 241
+__device__ __forceinline__ void dep_few(const DepositArgs& c, const unsigned* key, const unsigned* rec, const double* pack,
+                                        const long* bins, int cap, int b, int ntx, int nty, double* B) {
+    const int lane = threadIdx.x & 63;
+    const long lo = bins[2 * (long(cap) + b)];
+    const int m = int(bins[2 * (long(cap) + b) + 1] - lo);
+    const unsigned k = key[lo];
+    const int tile = int(k % unsigned(ntx * nty)), hw = int(k / unsigned(ntx * nty));
+    const int x0 = (tile % ntx) * kDT, y0 = (tile / ntx) * kDT;
+    if (lane < m) {
+        const double2* q = reinterpret_cast<const double2*>(pack + kDepPack * long(rec[lo + lane] / kDepSlots));
+        const double2 q0 = q[0], q1 = q[1], q2 = q[2];
+        int ix[3], jn[3]; double wx[3], wn[3];
+        tsc_w(q0.x, ix, wx);
+        tsc_w(q0.y, jn, wn);
+        double* r = B + kFewRec * lane;
+#pragma unroll
+        for (int u = 0; u < 3; ++u) { r[u] = q1.x * wx[u]; r[3 + u] = wn[u]; }
+        r[6] = q1.y; r[7] = q2.x; r[8] = q2.y; r[9] = 1 / q2.y;
+        reinterpret_cast<int2*>(r + 10)[0] = make_int2(wrap_index(ix[0], c.nx), wrap_index(jn[0], c.ny));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int x = x0 + (lane & (kDT - 1)), y = y0 + lane / kDT;
+    double a0 = 0, a1 = 0, a2 = 0;
+    // no branch: a particle that misses the cell adds zero, which never changes a sum that began as +0
+#pragma unroll 4
+    for (int t = 0; t < m; ++t) {
+        const double* r = B + kFewRec * t;
+        const int2 n0 = reinterpret_cast<const int2*>(r + 10)[0];
+        int u = x - n0.x, v = y - n0.y;
+        u += u < 0 ? c.nx : 0;
+        v += v < 0 ? c.ny : 0;
+        const bool in = u < 3 && v < 3;
+        const double w = r[in ? u : 0] * r[3 + (in ? v : 0)] * c.ia[0], vz = r[8], rz = r[9];
+        const double p0 = div_by(w * r[6], vz, rz), p1 = div_by(w * r[7], vz, rz);
+        a0 += in ? p0 : 0.0;
+        a1 += in ? p1 : 0.0;
+        a2 += in ? w : 0.0;
+    }
+    double* J = c.J + long(hw) * c.nk + long(y) * c.nx + x;
+    const long pl = long(c.nh) * c.nk;
+    J[0] = a0; J[pl] = a1; J[2 * pl] = a2;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();                  // before the next bin's records
+}
+// One workgroup per bin (persistent), then the bins of few.  A chunk of kDepLanes particles at a time, in list order: which of the tile's 8
 // columns and 8 rows a particle's stencil covers, as ballots over the wave; the product of a column's and a row's ballot
 // is the set of the cell's particles, so its population below a lane is the particle's rank in the cell's list.
 // Every record goes to its place in the list of its cell in LDS, and wave k < 3 adds component k, one lane per cell,
@@ -399,68 +453,9 @@ __global__ void __launch_bounds__(kDepLanes) k_dep_tile(DepositArgs c, const uns
             c.J[(long(wv) * c.nh + hw) * c.nk + long(y0 + lane / kDT) * c.nx + x0 + (lane & (kDT - 1))] = acc;
         __syncthreads();                              // before the next bin's ballots and lists
     }
-}
-
-// The bins of few particles, a wave each: the particles' stencils formed by a lane each and left in LDS, then one lane per
-// cell of the tile takes the particles in list order (a chain of kDepFew records, about a chunk of k_dep_tile).  That
-// kernel's workgroup fills a CU with its lists, so it takes 256 bins at a time however few their particles: electrons
-// anywhere in 128 slices of 16 x 512 points, all of g3d_bunch_currents, with the tiles alone, now, and by the record sort
-// (8 x 1024 points): 16384 electrons 441, 125 and 168 us; 65536 538, 178 and 288; 2^18 565, 292 and 440; 10^5 in 256 x 256
-// 2580 and 590.  A bunch pays a launch: 65536 166 -> 170 us, 2^18 233 -> 237.  kDepFew 16: 2^18 anywhere 453 us; 64:
-// 268, but the bunches 174 and 241.
-constexpr int kFewWaves = 4;                         // bins of a workgroup at a time
-constexpr int kFewRec = 11;                          // doubles per particle: f w_x (3), w_y (3), v_x, v_y, v_z, 1/v_z, first nodes
-__global__ void __launch_bounds__(64 * kFewWaves) k_dep_wave(DepositArgs c, const unsigned* key, const unsigned* rec,
-                                                             const double* pack, const long* bins, const int* cnt, int cap,
-                                                             int ntx, int nty) {
-    __shared__ double buf[kFewWaves][kDepFew * kFewRec];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    double* B = buf[wv];
-    const int nb = cnt[2];
-    for (int b = blockIdx.x * kFewWaves + wv; b < nb; b += gridDim.x * kFewWaves) {
-        const long lo = bins[2 * (long(cap) + b)];
-        const int m = int(bins[2 * (long(cap) + b) + 1] - lo);
-        const unsigned k = key[lo];
-        const int tile = int(k % unsigned(ntx * nty)), hw = int(k / unsigned(ntx * nty));
-        const int x0 = (tile % ntx) * kDT, y0 = (tile / ntx) * kDT;
-        if (lane < m) {
-            const double2* q = reinterpret_cast<const double2*>(pack + kDepPack * long(rec[lo + lane] / kDepSlots));
-            const double2 q0 = q[0], q1 = q[1], q2 = q[2];
-            int ix[3], jn[3]; double wx[3], wn[3];
-            tsc_w(q0.x, ix, wx);
-            tsc_w(q0.y, jn, wn);
-            double* r = B + kFewRec * lane;
-#pragma unroll
-            for (int u = 0; u < 3; ++u) { r[u] = q1.x * wx[u]; r[3 + u] = wn[u]; }
-            r[6] = q1.y; r[7] = q2.x; r[8] = q2.y; r[9] = 1 / q2.y;
-            reinterpret_cast<int2*>(r + 10)[0] = make_int2(wrap_index(ix[0], c.nx), wrap_index(jn[0], c.ny));
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int x = x0 + (lane & (kDT - 1)), y = y0 + lane / kDT;
-        double a0 = 0, a1 = 0, a2 = 0;
-        // no branch: a particle that misses the cell adds zero, which never changes a sum that began as +0
-#pragma unroll 4
-        for (int t = 0; t < m; ++t) {
-            const double* r = B + kFewRec * t;
-            const int2 n0 = reinterpret_cast<const int2*>(r + 10)[0];
-            int u = x - n0.x, v = y - n0.y;
-            u += u < 0 ? c.nx : 0;
-            v += v < 0 ? c.ny : 0;
-            const bool in = u < 3 && v < 3;
-            const double w = r[in ? u : 0] * r[3 + (in ? v : 0)] * c.ia[0], vz = r[8], rz = r[9];
-            const double p0 = div_by(w * r[6], vz, rz), p1 = div_by(w * r[7], vz, rz);
-            a0 += in ? p0 : 0.0;
-            a1 += in ? p1 : 0.0;
-            a2 += in ? w : 0.0;
-        }
-        double* J = c.J + long(hw) * c.nk + long(y) * c.nx + x;
-        const long pl = long(c.nh) * c.nk;
-        J[0] = a0; J[pl] = a1; J[2 * pl] = a2;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();              // before the next bin's records
-    }
+    // the bins of few particles too, a wave each, from the last workgroup (which had no other bin) on
+    for (int b = (int(gridDim.x) - 1 - int(blockIdx.x)) * kDepWaves + wv; b < cnt[2]; b += int(gridDim.x) * kDepWaves)
+        dep_few(c, key, rec, pack, bins, cap, b, ntx, nty, &vals[0][0] + wv * (kDepFew * kFewRec));
 }
 
 // Every buffer by its own length: the two sorts share some of them, and each needs other lengths of them
@@ -504,8 +499,6 @@ void tiled_deposit_run(const DepositArgs& a, Parts p, long np, unsigned nbin, De
                        s.nruns.data(), cap);
     hipLaunchKernelGGL(k_dep_tile, dim3(unsigned(std::min(cap, 1024))), dim3(kDepLanes), 0, stream(), a, s.k1.data(),
                        s.rec1.data(), s.val.data(), s.runs.data(), s.nruns.data(), cap, ntx, nty);
-    hipLaunchKernelGGL(k_dep_wave, dim3(std::min(blocks_for(cap, kFewWaves), 2048u)), dim3(64 * kFewWaves), 0, stream(), a,
-                       s.k1.data(), s.rec1.data(), s.val.data(), s.runs.data(), s.nruns.data(), cap, ntx, nty);
     launch_check("beam deposit (tiles)");
 }
 }  // namespace
