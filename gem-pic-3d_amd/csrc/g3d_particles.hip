@@ -265,8 +265,11 @@ __global__ void __launch_bounds__(kT) k_bunch_push(PushArgs c, Parts P, long np,
 // then waits on LDS instead of memory)
 constexpr int kBT = 8, kBM = 1, kBW = kBT + 3 + 2 * kBM, kBChunk = 1024;
 constexpr unsigned long long kBNone = ~0ull;
-// radix passes at every length (the default merges up to 2^20 records: 16 launches and 94 us for 2^18)
+// Long lists by radix passes: the default merges up to 2^20 records (16 launches for 2^18).  The push of 8000 electrons in
+// 256 slices of 64 x 64, by radix passes and merged, 100 and 69 us, 32000 121 and 97, 65000 153 and 131, 131000 165 and 157,
+// 2^18 192 and 227
 using BpushSort = rocprim::radix_sort_config<rocprim::default_config, rocprim::default_config, rocprim::default_config, 0>;
+constexpr long kBpushMerge = 1L << 17;               // records up to which the default is used
 
 // the bin of every particle that moves (alive 1 or 3, not frozen); the bin nbin (no window) for one outside the
 // slices of F; ~0 for the others (a frozen bunch particle only takes the new z here, as the plain push does)
@@ -940,13 +943,17 @@ void bunch_push_windowed(const PushArgs& a, Parts p, long np, double s0, BpushSc
     if (s.nchunk.size() < 1) s.nchunk.resize(1);
     hipLaunchKernelGGL(k_bpush_keys, dim3(blocks_for(np, kT)), dim3(kT), 0, stream(), a, p, np, ntx, nty, nbin,
                        s.key0.data(), s.idx0.data());
-    size_t bytes = 0;
-    hip_check(rocprim::radix_sort_pairs<BpushSort>(nullptr, bytes, s.key0.data(), s.key1.data(), s.idx0.data(), s.idx1.data(),
-                                        np, 0, unsigned(eb), stream()), "beam push sort size");
-    if (s.tmp.size() < bytes) s.tmp.resize(bytes + bytes / 4 + 256);
-    bytes = s.tmp.size();
-    hip_check(rocprim::radix_sort_pairs<BpushSort>(s.tmp.data(), bytes, s.key0.data(), s.key1.data(), s.idx0.data(),
-                                        s.idx1.data(), np, 0, unsigned(eb), stream()), "beam push sort");
+    auto sort = [&](auto config) {
+        size_t bytes = 0;
+        hip_check(rocprim::radix_sort_pairs<decltype(config)>(nullptr, bytes, s.key0.data(), s.key1.data(), s.idx0.data(),
+                                                              s.idx1.data(), np, 0, unsigned(eb), stream()), "beam push sort size");
+        if (s.tmp.size() < bytes) s.tmp.resize(bytes + bytes / 4 + 256);
+        bytes = s.tmp.size();
+        hip_check(rocprim::radix_sort_pairs<decltype(config)>(s.tmp.data(), bytes, s.key0.data(), s.key1.data(), s.idx0.data(),
+                                                              s.idx1.data(), np, 0, unsigned(eb), stream()), "beam push sort");
+    };
+    if (np <= kBpushMerge) sort(rocprim::default_config{});
+    else sort(BpushSort{});
     hip_check(hipMemsetAsync(s.nchunk.data(), 0, sizeof(int), stream()), "hipMemsetAsync");
     hipLaunchKernelGGL(k_bpush_chunks, dim3(blocks_for(np, kT)), dim3(kT), 0, stream(), s.key1.data(), np,
                        s.chunk.data(), s.nchunk.data(), cap);
